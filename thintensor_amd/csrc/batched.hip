@@ -1,9 +1,10 @@
 // Batched small-M dequant GEMM: y[m] = W x[m] for M activation rows.
 //
-//   * M below the MFMA threshold (int4: 4, fp8: 16): the GEMV engine with up to four
+//   * M below the fp16 MFMA threshold (int4: 4, fp8: 16): every row has the bits of the
+//     single-row GEMV.  fp8 M >= 3 runs on the binary32 matrix cores (rows_mfma.hip); M = 2,
+//     int4 M = 3 and operands past its 32-bit offsets run the GEMV engine with up to four
 //     activation rows per wave (every weight word decoded once, one fma chain per
-//     activation row), so row m equals the single-row GEMV bit for bit (one int4 row
-//     goes to the single-row kernel itself);
+//     activation row); one int4 or fp8 row goes to the single-row kernel itself;
 //   * from the threshold (int4 M >= 4, where the engine's per-row fma chains make it
 //     VALU-bound; fp8 M >= 16): MFMA (mfma_ksplit_kernel below): one workgroup per CU
 //     owns a block of weight rows for all M (<= 64) activation rows, its four waves
@@ -11,12 +12,10 @@
 //     operand registers, and the waves' fp32 tiles are summed in a fixed order at the
 //     end.  MFMA sums products in a hardware-defined order, so this path matches the
 //     dequantise-then-matmul reference to the stated tolerance, not bit for bit.
-//   * the M-row lm_head argmax runs the GEMV engine with eight activation rows per
-//     launch and one argmax key per (wave, row); a finishing kernel picks each row's
-//     token, as tt_matvec_argmax does for one row;
-//   * the M-row dense GEMV + bias of a batched decode step (tt_matvec_bias_rows, fp16)
-//     runs the same engine with eight rows per launch: each weight load feeds every
-//     row's fma chain, the bits per row those of the single-row operator.
+//   * the M-row lm_head argmax and the M-row dense GEMV + bias of a batched decode step
+//     (tt_matvec_bias_rows, fp16) run on the binary32 matrix cores from three rows on, each
+//     row with the bits of the single-row operator; below that the GEMV engine, with one
+//     argmax key per (wave, row) and a finishing kernel that picks each row's token.
 #include "gemv_impl.h"
 
 #include <type_traits>
@@ -615,10 +614,8 @@ int launch_mfma(MfmaParams P, hipStream_t st, const char* what) {
   return rc ? rc : check_launch(what);
 }
 
-// Up to four activation rows per GEMV launch, eight with M8 (the dense decode-step
-// GEMVs, whose fp16 weights are the largest reads of a batched step); VALU, bit-exact
-// per row.
-template <Fmt F, SMode SM, typename ST, int ROWS, int L, bool AM, bool M8 = AM>
+// Up to four activation rows per GEMV launch; VALU, bit-exact per row.
+template <Fmt F, SMode SM, typename ST, int ROWS, int L, bool AM>
 int launch_rows(GemvParams P, int64_t m_total, int64_t x_row, int64_t out_row, int lpr, hipStream_t st,
                 const char* what, int64_t partial_stride) {
   P.x_slot = x_row;
@@ -628,17 +625,13 @@ int launch_rows(GemvParams P, int64_t m_total, int64_t x_row, int64_t out_row, i
   uint64_t* part0 = P.am_partials;
   for (int64_t m0 = 0; m0 < m_total;) {
     const int64_t left = m_total - m0;
-    const int mr = (M8 && left >= 8) ? 8 : (left >= 4 ? 4 : (left >= 2 ? 2 : 1));
+    const int mr = left >= 4 ? 4 : (left >= 2 ? 2 : 1);
     GemvParams Q = P;
     Q.x = x0 + m0 * x_row;
     if (out0) Q.seg[0].out = out0 + m0 * out_row * 2;
     if (AM) Q.am_partials = part0 + m0 * partial_stride;
     int rc;
     switch (mr) {
-      case 8:
-        if constexpr (M8) rc = launch_lpr<F, SM, f16_t, f16_t, ST, ROWS, L, Pro::kLoad, false, 1, 8>(lpr, Q, 1, st, what);
-        else rc = TT_ERR_INVALID;
-        break;
       case 4: rc = launch_lpr<F, SM, f16_t, f16_t, ST, ROWS, L, Pro::kLoad, false, 1, 4>(lpr, Q, 1, st, what); break;
       case 2: rc = launch_lpr<F, SM, f16_t, f16_t, ST, ROWS, L, Pro::kLoad, false, 1, 2>(lpr, Q, 1, st, what); break;
       default: rc = launch_lpr<F, SM, f16_t, f16_t, ST, ROWS, L, Pro::kLoad, false, 1, 1>(lpr, Q, 1, st, what); break;
@@ -649,32 +642,20 @@ int launch_rows(GemvParams P, int64_t m_total, int64_t x_row, int64_t out_row, i
   return TT_OK;
 }
 
-// Token of each activation row.  Rows go to GEMV launches of eight (then four, two
-// and one for the tail); the launch holding rows m0 .. m0 + mr - 1 writes the key of
+// Token of each activation row.  Rows go to GEMV launches of four (then two and one for
+// the tail); the launch holding rows m0 .. m0 + mr - 1 writes the key of
 // (wave w, row r) at partials[m0 * per + w * mr + r].
 __global__ __launch_bounds__(256) void argmax_rows_kernel(const uint64_t* partials, int64_t per, int64_t m_total,
                                                           int64_t* out_idx, float* out_val) {
   const int64_t m = blockIdx.x;
-  int64_t b = m_total / 8 * 8, rem = m_total - b;
-  int64_t m0, mr;
+  const int64_t b = m_total / 4 * 4, rem = m_total - b;
+  int64_t m0 = m, mr = 1;
   if (m < b) {
-    m0 = m / 8 * 8;
-    mr = 8;
-  } else {
-    if (rem >= 4 && m >= b + 4) {
-      b += 4;
-      rem -= 4;
-    }
-    if (rem >= 4) {
-      m0 = b;
-      mr = 4;
-    } else if (rem >= 2 && m < b + 2) {
-      m0 = b;
-      mr = 2;
-    } else {
-      m0 = m;
-      mr = 1;
-    }
+    m0 = m / 4 * 4;
+    mr = 4;
+  } else if (rem >= 2 && m < b + 2) {
+    m0 = b;
+    mr = 2;
   }
   const uint64_t* base = partials + m0 * per + (m - m0);
   __shared__ uint64_t red[256];
@@ -710,6 +691,8 @@ __global__ __launch_bounds__(256) void argmax_rows_kernel(const uint64_t* partia
 namespace tt {
 int dense_bias_rows_f16(const void* weight, int64_t w_row, const void* bias, const void* x, int64_t x_row, void* out,
                         int64_t out_row, int64_t m, int64_t rows, int64_t cols, hipStream_t st) {
+  if (m >= kRowsMfmaMin && rows_mfma_fits(w_row * 2, x_row))
+    return rows_mfma_f16({weight, w_row * 2, nullptr, bias, x, x_row, out, out_row, m, rows, cols}, st, "matvec_bias_rows");
   GemvParams P{};
   P.nseg = 1;
   P.seg[0] = Seg{static_cast<const uint8_t*>(weight), w_row * 2, nullptr, 0, 0, out, (int)rows};
@@ -717,7 +700,7 @@ int dense_bias_rows_f16(const void* weight, int64_t w_row, const void* bias, con
   P.x = x;
   P.cols = (int)cols;
   const int lpr = tt_gemv_lanes_per_row(cols / 32, 1);
-  return launch_rows<Fmt::kF16W, SMode::kNone, float, 2, 1, false, true>(P, m, x_row, out_row, lpr, st,
+  return launch_rows<Fmt::kF16W, SMode::kNone, float, 2, 1, false>(P, m, x_row, out_row, lpr, st,
                                                                          "matvec_bias_rows", 0);
 }
 }  // namespace tt
@@ -788,6 +771,8 @@ extern "C" int tt_scaled_batched_matvec(const void* weight, int64_t w_row_bytes,
                  static_cast<uint16_t*>(out), out_row, (int)m, (int)rows, (int)cols};
     return launch_mfma<WFmt::kFp8Row>(P, st, what);
   }
+  if (m >= kRowsMfmaMin && rows_mfma_fits(w_row_bytes, x_row))
+    return rows_mfma_fp8({weight, w_row_bytes, scales, nullptr, x, x_row, out, out_row, m, rows, cols}, st, what);
   if (m == 1)   // one row: the single-row GEMV itself (its lean kernel; the same bits as a row of the engine)
     return tt_scaled_matvec(weight, TT_W_FP8, w_row_bytes, scales, TT_F32, x, TT_F16, out, TT_F16, rows, cols, stream);
   GemvParams P{};
@@ -816,6 +801,10 @@ extern "C" int tt_matvec_argmax_batched(const void* weight, int64_t w_row, const
   TT_REQUIRE(logits == nullptr || logits_row >= rows, "%s: bad logits stride", what);
   const int64_t per = tt_matvec_argmax_partials(rows, cols);
   TT_REQUIRE(partials_capacity >= m * per, "%s: partials buffer needs %lld entries", what, (long long)(m * per));
+  if (m >= kRowsMfmaMin && rows_mfma_fits(w_row * 2, x_row))
+    return rows_mfma_argmax_f16({weight, w_row * 2, nullptr, nullptr, x, x_row, logits, logits ? logits_row : 0, m, rows,
+                                 cols, partials, per},
+                                out_idx, out_val, static_cast<hipStream_t>(stream), what);
   GemvParams P{};
   P.nseg = 1;
   P.seg[0] = Seg{static_cast<const uint8_t*>(weight), w_row * 2, nullptr, 0, 0, logits, (int)rows};

@@ -139,7 +139,10 @@ extern "C" int tt_matvec_bias_rows(const void* weight, int w_dtype, int64_t w_ro
     return TT_OK;
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (w_dtype == TT_F16 && x_dtype == TT_F16 && cols <= 4096)   // eight activation rows in 64 KB of LDS
+  // the GEMV engine takes up to 4096 columns (its activation rows share LDS), the matrix-core
+  // kernel any width
+  if (w_dtype == TT_F16 && x_dtype == TT_F16 &&
+      (cols <= 4096 || (m >= kRowsMfmaMin && rows_mfma_fits(w_row * 2, x_row))))
     return dense_bias_rows_f16(weight, w_row, bias, x, x_row, out, out_row, m, rows, cols, st);
   // rows of the batch are slots of the lean kernel (blockIdx.y), each with its own
   // activation and output row; the arithmetic per row is the single-row kernel's

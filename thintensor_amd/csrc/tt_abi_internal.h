@@ -40,11 +40,42 @@ inline int check_launch(const char* what) {
 
 inline bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
 
-// y[r] = W x[r] + bias for m fp16 activation rows through the GEMV engine, several rows
-// per launch sharing every weight load; row r has the bits of the single-row GEMV + bias
-// (batched.hip).  Shapes and alignment checked by the caller.
+// y[r] = W x[r] + bias for m fp16 activation rows, several rows per launch sharing every
+// weight load; row r has the bits of the single-row GEMV + bias (batched.hip).  Shapes and
+// alignment checked by the caller.
 int dense_bias_rows_f16(const void* weight, int64_t w_row, const void* bias, const void* x, int64_t x_row, void* out,
                         int64_t out_row, int64_t m, int64_t rows, int64_t cols, hipStream_t st);
+
+// y[r] = W x[r] for m fp16 activation rows on the binary32 matrix cores, row r with the
+// bits of the single-row GEMV (rows_mfma.hip): fp16 weights with an optional fp16 bias, fp8
+// weights with fp32 row scales, and the fp16 lm_head with its argmax.  Passes of kRowsPass
+// rows.  Shapes (cols a multiple of 32) and 16-byte alignment checked by the caller.
+constexpr int kRowsPass = 32;
+// Smallest M of the fp16 GEMVs and of the fp8 GEMM that runs there (same bits as the GEMV
+// engine).  Three rows take the engine two launches (fp16 152064 x 5120 522 us against 263,
+// fp8 17920 x 5120 39 against 24); at two, one launch each, the engine is as fast or faster
+// (268 against 263 us, 18.8 against 21.2).
+constexpr int kRowsMfmaMin = 3;
+struct RowsArgs {
+  const void* weight;
+  int64_t w_row_bytes;
+  const float* scales;
+  const void* bias;
+  const void* x;
+  int64_t x_row;
+  void* out;
+  int64_t out_row;
+  int64_t m, rows, cols;
+  uint64_t* keys;         // argmax scratch, keys_per_row entries per activation row
+  int64_t keys_per_row;
+};
+// 32-bit byte offsets inside a weight tile (32 rows) and an activation pass
+inline bool rows_mfma_fits(int64_t w_row_bytes, int64_t x_row) {
+  return w_row_bytes < (1LL << 26) && x_row < (1LL << 25);
+}
+int rows_mfma_f16(const RowsArgs& A, hipStream_t st, const char* what);
+int rows_mfma_fp8(const RowsArgs& A, hipStream_t st, const char* what);
+int rows_mfma_argmax_f16(const RowsArgs& A, int64_t* out_idx, float* out_val, hipStream_t st, const char* what);
 
 // Expert index arrays are int32 or int64 (index_bytes 4 or 8); the kernels take the
 // log2 of the size in 32-bit words.
