@@ -295,3 +295,40 @@ def test_fp8_full_size_relative_error(device):
     normal = y.abs() >= 2.0 ** -6
     assert bool(((d - y).abs() <= y.abs() * 2.0 ** -4 + 1e-30)[normal].all())
     assert float(d.abs().max()) == 448.0
+
+
+@pytest.mark.parametrize("mode", ["lsq", "rows"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows,cols,group", [(1, 8, 32), (3, 40, 32), (7, 1000, 512), (130, 520, 64), (5, 34, 64),
+                                             (2049, 2048, 256)])
+def test_int4_symmetric_edges(affine_env, mode, dtype, rows, cols, group):
+    """The eight-elements-per-lane kernel (and the one-wave-per-group kernel at width 34)
+    at its edges: ragged last groups, one piece, four pieces per thread, exact ties of
+    x / scale, all-zero groups, values below 1e-12.  With infinities and NaN, which the
+    oracle's numpy folds treat differently, the two kernels against each other: a source
+    that is not 16-byte aligned takes the one-wave-per-group kernel."""
+    affine_env(False)
+    g = torch.Generator().manual_seed(rows + cols)
+    w = torch.randn((rows, cols), generator=g) * 0.02
+    w[::4] = torch.randint(-14, 15, (len(w[::4]), cols), generator=g).float() * 0.5      # ties at scale 1
+    if rows > 2:
+        w[2, ::5] = 1e-13
+        w[2, 1::5] = 0
+        w[1, : cols // 2] = 0
+    call, oracle_of = (TQ.quantize_to_int4_cpu, Q.int4_lsq) if mode == "lsq" else (TQ.quantize_int4_rows, Q.int4_rows)
+    src = w.to(dtype)
+    got = call(src.cuda(), group_size=group)
+    want = oracle_of(src.float().numpy(), group)
+    eq(got[0], want[0], "codes")
+    eq(got[1], want[1].view(np.uint16) if mode == "lsq" else want[1], "scales")
+    m = torch.rand((rows, cols), generator=g)
+    for lo, v in ((0.0, float("inf")), (0.01, float("-inf")), (0.02, float("nan"))):
+        src[(m >= lo) & (m < lo + 0.002)] = v
+    src[0, 0] = float("inf")
+    got = call(src.cuda(), group_size=group)
+    shifted = torch.empty(rows * cols + 1, device="cuda", dtype=dtype)[1:].view(rows, cols)
+    shifted.copy_(src)
+    want = call(shifted, group_size=group)
+    eq(got[0], as_np(want[0]), "codes with infinities")
+    eq(got[1].view(torch.int16 if mode == "lsq" else torch.int32), as_np(want[1].view(torch.int16 if mode == "lsq" else torch.int32)),
+       "scales with infinities")

@@ -137,8 +137,158 @@ struct Q4Params {
   int rows, cols, group, groups;
 };
 
-// One wave per (row, group).  Lane l holds elements [l * EPL, (l + 1) * EPL) of the
-// group (EPL = G / 64), or element l for G = 32.
+// Symmetric INT4 (kLsq, kRows) for widths that are a multiple of eight and 16-byte aligned
+// rows: eight consecutive elements per lane, GL = G / 8 lanes per group, 64 / GL groups per
+// wave, up to kQ4Pieces pieces per thread requested before the first is used (one while the
+// grid is small: 512 x 1024 fp16 5.0 us with four, 2.8 with one; one wave per
+// group 3.7).
+//
+// The sums need no particular order here.  A nonzero code means |x| >= amax / 14, so every
+// nonzero product x q lies within 2^4 of the largest x: with 24-bit products the sum over 512
+// elements spans at most 9 + 3 + 4 + 24 = 40 bits and is exact in binary64, and with 11-bit
+// sources the sum over a lane's eight elements spans 3 + 3 + 5 + 10 = 21 bits and is exact in
+// binary32.  (NaN and infinite elements give NaN in every order.)
+//
+// rint(x / s) is taken from x * rcp(s) unless that lies within 1e-5 of a half-integer (or is
+// not finite): product (rcp is good to one ulp below 2^126, where its result is normal) and
+// quotient are both within 3e-6 of the true value while it is below 9, past which both clamp
+// alike.  A lane that is closer divides, its wave with it (bf16 sources often: x / amax is
+// then an odd multiple of 1 / 14 for some x of every seventh amax).
+//
+// Bound by HBM and the vector units about equally.  17920 x 5120 bf16, group 128: one wave
+// per group with binary64 folds over 64 lanes and two divisions per element 280 -> 89 us on
+// fresh buffers (2.6 TB/s; fp16 74 us, fp32 250 -> 82 us; group 32, half of whose waves'
+// lanes idled, fp16 855 -> 60 us).
+constexpr int kQ4Pieces = 4;
+
+template <int GL, typename T, typename F>
+__device__ __forceinline__ T fold_lanes(T v, F&& op) {
+  if constexpr (GL > 1) v = op(v, std::integral_constant<int, 1>{});
+  if constexpr (GL > 2) v = op(v, std::integral_constant<int, 2>{});
+  if constexpr (GL > 4) v = op(v, std::integral_constant<int, 4>{});
+  if constexpr (GL > 8) v = op(v, std::integral_constant<int, 8>{});
+  if constexpr (GL > 16) v = op(v, std::integral_constant<int, 16>{});
+  if constexpr (GL > 32) v = op(v, std::integral_constant<int, 32>{});
+  return v;
+}
+
+// rint(x / s), clamped to [lo, 7] with CLAMP.  NaN and infinite quotients come out alike on
+// both paths, so the maximum may skip their NaN distances.
+template <bool CLAMP>
+__device__ __forceinline__ void round_codes(const float (&x)[8], float s, float lo, float (&q)[8]) {
+  const float r = __builtin_amdgcn_rcpf(s);
+  float far = 0.0f;   // largest distance of a product from its nearest integer
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    const float t = x[k] * r;
+    const float n = __builtin_rintf(t);
+    far = fmaxf(far, fabsf(t - n));
+    q[k] = CLAMP ? clampf(n, lo, 7.0f) : n;
+  }
+  if (far > 0.49999f || !(s < 0x1p126f)) {
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      const float n = __builtin_rintf(x[k] / s);
+      q[k] = CLAMP ? clampf(n, lo, 7.0f) : n;
+    }
+  }
+}
+
+// NP pieces per thread.  Offsets inside a workgroup's rows are 32-bit (checked by the host).
+template <typename ST, int GL, bool LSQ, int NP>
+__global__ __launch_bounds__(256) void int4_sym_kernel(const Q4Params P, int ppr) {
+  constexpr int kQuads = sizeof(ST) == 4 ? 2 : 1;
+  typedef uint32_t quad_t __attribute__((ext_vector_type(4)));
+  // pieces of eight elements, ppr of them per row (whole groups); those past the width or
+  // the last row are read at a valid place and count as absent
+  const int64_t base = (int64_t)blockIdx.x * (256 * NP);
+  const int64_t row0 = base / ppr;
+  const uint32_t rem0 = (uint32_t)(base - row0 * ppr) + threadIdx.x;
+  const uint32_t rows_left = P.rows - row0 < (1 << 20) ? (uint32_t)(P.rows - row0) : 1u << 20;
+  const uint32_t width = (uint32_t)P.cols >> 3;
+  const ST* src = reinterpret_cast<const ST*>(P.src) + row0 * P.src_row;
+  uint8_t* packed = P.packed + row0 * (P.cols >> 1);
+  quad_t raw[NP][kQuads];
+  uint32_t dr[NP], piece[NP];
+#pragma unroll
+  for (int i = 0; i < NP; i++) {
+    const uint32_t rem = rem0 + 256 * i;
+    dr[i] = rem / (uint32_t)ppr;
+    piece[i] = rem - dr[i] * ppr;
+    const uint32_t lr = dr[i] < rows_left ? dr[i] : rows_left - 1;
+    const uint32_t lp = piece[i] < width ? piece[i] : width - 1;
+    const quad_t* p = reinterpret_cast<const quad_t*>(reinterpret_cast<const uint8_t*>(src) +
+                                                      (lr * (uint32_t)P.src_row + lp * 8) * (uint32_t)sizeof(ST));
+#pragma unroll
+    for (int h = 0; h < kQuads; h++) raw[i][h] = p[h];
+  }
+  __builtin_amdgcn_sched_barrier(0);   // every piece requested before the first is used
+#pragma unroll
+  for (int i = 0; i < NP; i++) {
+    const bool on = dr[i] < rows_left && piece[i] < width;
+    float x[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      if constexpr (sizeof(ST) == 4) {
+        const uint32_t w = on ? raw[i][k >> 2][k & 3] : 0u;
+        x[k] = __builtin_bit_cast(float, w);
+      } else {
+        const uint32_t w = on ? raw[i][0][k >> 1] : 0u;
+        x[k] = (k & 1) ? hi_f32<ST>(w) : lo_f32<ST>(w);
+      }
+    }
+    float amax = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; k++) amax = fmaxf(amax, fabsf(x[k]));
+    amax = fold_lanes<GL>(amax, [](float v, auto m) { return fmaxf(v, xor_partner<decltype(m)::value>(v)); });
+    float s = fmaxf(amax, kTiny) / 7.0f;
+    float q[8];
+    if constexpr (!LSQ) {
+      round_codes<true>(x, s, -7.0f, q);
+    } else {
+      // |x / s| <= 7 unless x is NaN or infinite; a NaN product makes the sum NaN whatever its
+      // code, an infinite one only with the clamped code
+      round_codes<false>(x, s, 0.0f, q);
+      if (amax == __builtin_inff()) {
+#pragma unroll
+        for (int k = 0; k < 8; k++) q[k] = clampf(q[k], -8.0f, 7.0f);
+      }
+      double num = 0.0;
+      float den = 0.0f;
+      if constexpr (sizeof(ST) == 4) {
+#pragma unroll
+        for (int k = 0; k < 8; k++) num = num + (double)(x[k] * q[k]);
+      } else {
+        float part = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 8; k++) part = __builtin_fmaf(x[k], q[k], part);
+        num = (double)part;
+      }
+#pragma unroll
+      for (int k = 0; k < 8; k++) den = __builtin_fmaf(q[k], q[k], den);
+      num = fold_lanes<GL>(num, [](double v, auto m) { return v + xor_partner_d<decltype(m)::value>(v); });
+      den = fold_lanes<GL>(den, [](float v, auto m) { return v + xor_partner<decltype(m)::value>(v); });
+      s = fmaxf(fabsf((float)num / fmaxf(den, 1.0f)), kTiny);
+      round_codes<true>(x, s, -8.0f, q);
+    }
+    // four codes + 8 as one exact binary32 number
+    const float lo4 = __builtin_fmaf(4096.0f, q[3], __builtin_fmaf(256.0f, q[2], __builtin_fmaf(16.0f, q[1], q[0]))) + 34952.0f;
+    const float hi4 = __builtin_fmaf(4096.0f, q[7], __builtin_fmaf(256.0f, q[6], __builtin_fmaf(16.0f, q[5], q[4]))) + 34952.0f;
+    if (on) {
+      *reinterpret_cast<uint32_t*>(packed + (dr[i] * ((uint32_t)P.cols >> 1) + piece[i] * 4)) =
+          (uint32_t)lo4 | ((uint32_t)hi4 << 16);
+      if ((threadIdx.x & (GL - 1)) == 0) {
+        const int64_t si = row0 * P.groups + (dr[i] * (uint32_t)P.groups + piece[i] / GL);
+        if constexpr (LSQ) reinterpret_cast<uint16_t*>(P.scales)[si] = f32_to_f16_bits(s);
+        else reinterpret_cast<float*>(P.scales)[si] = s;
+      }
+    }
+  }
+}
+
+// One wave per (row, group): the affine modes, and symmetric ones of other widths and
+// alignments.  Lane l holds elements [l * EPL, (l + 1) * EPL) of the group (EPL = G / 64), or
+// element l for G = 32.
 template <typename ST, int EPL, int MODE>
 __global__ __launch_bounds__(256) void int4_quant_kernel(const Q4Params P) {
   const int lane = threadIdx.x & 63;
@@ -642,6 +792,37 @@ extern "C" int tt_quantize_int4(const void* src, int src_dtype, int64_t rows, in
   const int groups = (int)((cols + group_size - 1) / group_size);
   Q4Params P{src, src_row, importance, gptq_factors, packed, scales, (int)rows, (int)cols, (int)group_size, groups};
   hipStream_t st = static_cast<hipStream_t>(stream);
+  const bool sym = mode == TT_Q4_LSQ || mode == TT_Q4_ROWS;
+  const int src_size = src_dtype == TT_F32 ? 4 : 2;
+  const int64_t ppr = groups * (group_size / 8);   // eight-element pieces per row, whole groups
+  // a workgroup of the vector kernel touches up to 256 kQ4Pieces / ppr + 2 rows, with 32-bit offsets
+  const int64_t span = src_row * src_size * (256 * kQ4Pieces / ppr + 2);
+  if (sym && cols % 8 == 0 && aligned(src, 16) && src_row * src_size % 16 == 0 && aligned(packed, 4) && span < (1ll << 31) &&
+      rows * ppr < (1ll << 31) * 256) {
+    const int64_t pieces = rows * ppr;
+    return by_src_dtype(src_dtype, what, [&](auto t) -> int {
+      using ST = decltype(t);
+      auto go = [&](auto gl) -> int {
+        constexpr int GL = decltype(gl)::value;
+        auto launch = [&](auto np) -> int {
+          constexpr int NP = decltype(np)::value;
+          const dim3 grid((unsigned)((pieces + 256 * NP - 1) / (256 * NP)));
+          if (mode == TT_Q4_LSQ) hipLaunchKernelGGL((int4_sym_kernel<ST, GL, true, NP>), grid, dim3(256), 0, st, P, (int)ppr);
+          else hipLaunchKernelGGL((int4_sym_kernel<ST, GL, false, NP>), grid, dim3(256), 0, st, P, (int)ppr);
+          return check_launch(what);
+        };
+        if (pieces < 256 * 2048) return launch(std::integral_constant<int, 1>{});
+        return launch(std::integral_constant<int, kQ4Pieces>{});
+      };
+      switch (group_size) {
+        case 32: return go(std::integral_constant<int, 4>{});
+        case 64: return go(std::integral_constant<int, 8>{});
+        case 128: return go(std::integral_constant<int, 16>{});
+        case 256: return go(std::integral_constant<int, 32>{});
+        default: return go(std::integral_constant<int, 64>{});
+      }
+    });
+  }
   const int64_t waves = rows * groups;
   TT_REQUIRE((waves + 3) / 4 < (1ll << 31), "%s: too many groups", what);
   const dim3 grid((unsigned)((waves + 3) / 4));
