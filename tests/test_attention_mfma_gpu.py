@@ -1,0 +1,57 @@
+"""Decode attention outside the one-launch grids: matrix-core chunk partials and the fold
+(attn_mfma_kernel, attn_fold_kernel) bit for bit against the oracle, for every number of
+query heads per KV head, both head dimensions and KV types, capacities that end inside a
+chunk, strided caches, garbage past the count, one token and several fold blocks."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from tests.helpers import rng, to_torch
+from tests.test_gemv_gpu import assert_bits_equal
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,tokens,cap,bf16,sinks,pad", [
+    (40, 10, 128, 130, 200, True, False, 0),     # four heads per KV head, capacity inside a chunk
+    (2, 2, 128, 1, 1, False, True, 0),           # one head, one token, one-row cache
+    (6, 3, 128, 64, 64, True, True, 0),          # two heads, exactly one chunk
+    (8, 1, 64, 8257, 8300, False, True, 0),      # 130 chunks: a second fold block of two
+    (16, 1, 64, 2050, 2050, False, False, 0),    # sixteen heads, four waves
+    (16, 2, 128, 1041, 1100, True, False, 0),    # eight heads, 17 chunks
+    (264, 33, 64, 700, 704, False, False, 0),    # whole chunks, more workgroups than CUs
+    (4, 1, 64, 77, 100, True, False, 8),         # token stride above the head dimension
+    (4, 1, 96, 77, 128, False, True, 0),         # other head dimension: scalar loads
+    (4, 1, 64, 77, 128, False, False, 1),        # misaligned rows: scalar loads
+])
+def test_attention_partials_and_fold(backend, device, heads, kv_heads, dim, tokens, cap, bf16, sinks, pad):
+    g = rng(heads + tokens + dim)
+
+    def values(*shape):
+        v = g.standard_normal(shape).astype(np.float32)
+        if bf16:
+            return torch.from_numpy(v).to(torch.bfloat16).view(torch.int16).numpy().view(np.uint16)
+        return v.astype(np.float16)
+
+    q, sk = values(heads * dim), values(heads) if sinks else None
+    keys, vals = values(kv_heads, cap, dim + pad), values(kv_heads, cap, dim + pad)
+    code, dtype = (oracle.BF16, torch.bfloat16) if bf16 else (oracle.F16, torch.float16)
+    nan, inf = (0x7fc0, 0x7f80) if bf16 else (np.float16(np.nan), np.float16(np.inf))
+    keys[:, tokens:], vals[:, tokens:] = nan, inf             # past the count: never used
+    qd, kd, vd = (to_torch(a, device, bf16) for a in (q, keys, vals))
+    kd, vd = kd[:, :, :dim], vd[:, :, :dim]
+    skd = to_torch(sk, device, bf16) if sinks else None
+    out = torch.empty(heads * dim, device=device, dtype=dtype)
+    stride = (cap * (dim + pad), dim + pad)
+    for n, count in ((tokens, torch.tensor([tokens], dtype=torch.int32, device=device)), (max(1, tokens // 2), None)):
+        backend.single_token_gqa_attention(qd, kd, vd, out, heads, kv_heads, dim, sinks=skd,
+                                           active_tokens=n if count is None else count)
+        want = np.empty(heads * dim, dtype=q.dtype)
+        oracle.lib().tto_attention(q.ctypes.data, keys.ctypes.data, vals.ctypes.data, code, *stride, *stride,
+                                   sk.ctypes.data if sinks else None, code, n, heads, kv_heads, dim, want.ctypes.data)
+        got = out.cpu().view(torch.int16).numpy().view(np.uint16)
+        assert_bits_equal(got, want.view(np.uint16), f"{n} tokens")

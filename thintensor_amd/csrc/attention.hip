@@ -17,12 +17,14 @@
 // growing cache; chunks past the count exit without work.  The count is clamped to
 // max_tokens so a runaway device counter can never read past the cache.
 //
-// Contiguous head_dim-64 caches use kernels that issue every load before the first
-// wait: the chunk wave requests its K row, V column and query rows before the active
-// count is known (all rows up to the capacity are in bounds), and the combine wave
-// requests the chunk metadata and up to 32 chunks of partial outputs at once.
+// Three forms, all with these bits: one launch for small grids of contiguous head_dim-64
+// caches (attn_kvchunk_kernel), matrix-core partials and a fold for everything else of
+// head_dim 64 or 128 (attn_mfma_kernel, attn_fold_kernel), scalar loads for the rest
+// (attn_partial_kernel, attn_combine_kernel).
 #include "tt_abi_internal.h"
 #include "tt_common.h"
+
+#include <type_traits>
 
 namespace tt {
 
@@ -44,13 +46,10 @@ struct AttnParams {
   void* out;              // [heads, D]
 };
 
-// DC: head_dim known at compile time (0: runtime head_dim, scalar loads).  With DC
-// set and contiguous rows (token stride DC), the K row of a lane is read with
-// 128-bit loads and the V column of the chunk is loaded in full before the weighted
-// sum, so each phase waits for memory once.
-template <typename T, int G, int DC>
+// Any head_dim up to 256, strides and alignment: scalar loads.
+template <typename T, int G>
 __device__ void attn_chunk(const AttnParams& P, int kvh, int c, int T_act) {
-  const int D = DC ? DC : P.head_dim;
+  const int D = P.head_dim;
   const int lane = threadIdx.x;
   __shared__ float q_s[G * 256];
   __shared__ float p_s[G * kChunk];
@@ -64,39 +63,11 @@ __device__ void attn_chunk(const AttnParams& P, int kvh, int c, int T_act) {
   float sc[G];
 #pragma unroll
   for (int g = 0; g < G; g++) sc[g] = 0.0f;
-  // V column requested together with K when the registers allow it (G <= 4)
-  constexpr bool kVEarly = DC == 64 && G <= 4;
-  float vv[DC == 64 ? kChunk : 1];
-  if constexpr (DC != 0) {
-    // contiguous rows, capacity a whole number of chunks: every row of the chunk is in
-    // bounds, rows past the count are read and masked
-    const uint4* krow = reinterpret_cast<const uint4*>(reinterpret_cast<const T*>(P.keys) + kvh * P.k_head + (int64_t)t * DC);
-    uint4 kr[DC / 8];
+  const T* krow = reinterpret_cast<const T*>(P.keys) + kvh * P.k_head + (int64_t)(valid ? t : 0) * P.k_tok;
+  for (int d = 0; d < D; d++) {
+    const float kv = to_f32(krow[d]);
 #pragma unroll
-    for (int i = 0; i < DC / 8; i++) kr[i] = krow[i];
-    if constexpr (kVEarly) {
-      // the chunk's V column (lane = dimension) is requested together with K
-      const T* vcol = reinterpret_cast<const T*>(P.values) + kvh * P.v_head + (int64_t)(c * kChunk) * DC + lane;
-#pragma unroll
-      for (int tt = 0; tt < kChunk; tt++) vv[tt] = to_f32(vcol[tt * DC]);
-    }
-#pragma unroll
-    for (int i = 0; i < DC / 8; i++) {
-      const uint32_t kw[4] = {kr[i].x, kr[i].y, kr[i].z, kr[i].w};
-#pragma unroll
-      for (int e = 0; e < 8; e++) {
-        const float kv = (e & 1) ? hi_f32<T>(kw[e >> 1]) : lo_f32<T>(kw[e >> 1]);
-#pragma unroll
-        for (int g = 0; g < G; g++) sc[g] = __builtin_fmaf(q_s[g * DC + 8 * i + e], kv, sc[g]);
-      }
-    }
-  } else {
-    const T* krow = reinterpret_cast<const T*>(P.keys) + kvh * P.k_head + (int64_t)(valid ? t : 0) * P.k_tok;
-    for (int d = 0; d < D; d++) {
-      const float kv = to_f32(krow[d]);
-#pragma unroll
-      for (int g = 0; g < G; g++) sc[g] = __builtin_fmaf(q_s[g * D + d], kv, sc[g]);
-    }
+    for (int g = 0; g < G; g++) sc[g] = __builtin_fmaf(q_s[g * D + d], kv, sc[g]);
   }
   const float ninf = __builtin_bit_cast(float, 0xff800000u);
 #pragma unroll
@@ -120,47 +91,27 @@ __device__ void attn_chunk(const AttnParams& P, int kvh, int c, int T_act) {
   }
   __syncthreads();
   // phase 2: lane = dimension, o = fma chain over the chunk's tokens ascending
-  if constexpr (DC == 64) {
-    if constexpr (!kVEarly) {
-      const T* vcol = reinterpret_cast<const T*>(P.values) + kvh * P.v_head + (int64_t)(c * kChunk) * DC + lane;
-#pragma unroll
-      for (int tt = 0; tt < kChunk; tt++) vv[tt] = to_f32(vcol[tt * DC]);
-    }
+  for (int d = lane; d < D; d += 64) {
     float o[G];
 #pragma unroll
     for (int g = 0; g < G; g++) o[g] = 0.0f;
-    // tokens past the count add fma(0, 0, o) == o (p is 0 there and o is never -0)
+    const T* vcol = reinterpret_cast<const T*>(P.values) + kvh * P.v_head + (int64_t)(c * kChunk) * P.v_tok + d;
+    for (int tt = 0; tt < nt; tt++) {
+      const float vv = to_f32(vcol[(int64_t)tt * P.v_tok]);
 #pragma unroll
-    for (int tt = 0; tt < kChunk; tt++) {
-      const float v = tt < nt ? vv[tt] : 0.0f;
-#pragma unroll
-      for (int g = 0; g < G; g++) o[g] = __builtin_fmaf(p_s[g * kChunk + tt], v, o[g]);
+      for (int g = 0; g < G; g++) o[g] = __builtin_fmaf(p_s[g * kChunk + tt], vv, o[g]);
     }
 #pragma unroll
-    for (int g = 0; g < G; g++) P.part_o[((int64_t)(h0 + g) * P.max_chunks + c) * DC + lane] = o[g];
-  } else {
-    for (int d = lane; d < D; d += 64) {
-      float o[G];
-#pragma unroll
-      for (int g = 0; g < G; g++) o[g] = 0.0f;
-      const T* vcol = reinterpret_cast<const T*>(P.values) + kvh * P.v_head + (int64_t)(c * kChunk) * P.v_tok + d;
-      for (int tt = 0; tt < nt; tt++) {
-        const float vv = to_f32(vcol[(int64_t)tt * P.v_tok]);
-#pragma unroll
-        for (int g = 0; g < G; g++) o[g] = __builtin_fmaf(p_s[g * kChunk + tt], vv, o[g]);
-      }
-#pragma unroll
-      for (int g = 0; g < G; g++) P.part_o[((int64_t)(h0 + g) * P.max_chunks + c) * D + d] = o[g];
-    }
+    for (int g = 0; g < G; g++) P.part_o[((int64_t)(h0 + g) * P.max_chunks + c) * D + d] = o[g];
   }
 }
 
-template <typename T, int G, int DC>
+template <typename T, int G>
 __global__ __launch_bounds__(64) void attn_partial_kernel(AttnParams P) {
   const int kvh = blockIdx.y;
   const int c = blockIdx.x;
   const int T_act = min(P.tokens_dev ? P.tokens_dev[0] + P.tokens : P.tokens, P.max_tokens);
-  if (c * kChunk < T_act) attn_chunk<T, G, DC>(P, kvh, c, T_act);
+  if (c * kChunk < T_act) attn_chunk<T, G>(P, kvh, c, T_act);
 }
 
 // Combine of one head, same arithmetic as the sequential description above: the
@@ -234,345 +185,26 @@ __global__ __launch_bounds__(64) void attn_combine_kernel(AttnParams P) {
   combine_head<T, SKT>(P, blockIdx.x, threadIdx.x);
 }
 
-// Chunk partials for contiguous head_dim-64 caches whose capacity is a whole number
-// of chunks (every row of every chunk is in bounds, so all loads are issued before the
-// active count is known).  Same arithmetic as attn_chunk.
-template <typename T, int G>
-__global__ __launch_bounds__(64) void attn_partial64_kernel(AttnParams P) {
-  constexpr int D = 64;
-  const int kvh = blockIdx.y;
-  const int c = blockIdx.x;
-  const int lane = threadIdx.x;
-  const int h0 = kvh * G;
-  __shared__ float q_s[G * D];
-  __shared__ float p_s[G * kChunk];
-  // K row of this lane's token, the chunk's V column (lane = dimension), query rows
-  const int t = c * kChunk + lane;
-  const uint4* krow = reinterpret_cast<const uint4*>(reinterpret_cast<const T*>(P.keys) + kvh * P.k_head + (int64_t)t * D);
-  uint4 kr[D / 8];
-#pragma unroll
-  for (int i = 0; i < D / 8; i++) kr[i] = krow[i];
-  const T* vcol = reinterpret_cast<const T*>(P.values) + kvh * P.v_head + (int64_t)(c * kChunk) * D + lane;
-  T vraw[kChunk];
-#pragma unroll
-  for (int tt = 0; tt < kChunk; tt++) vraw[tt] = vcol[tt * D];
-  T qraw[G];
-#pragma unroll
-  for (int g = 0; g < G; g++) qraw[g] = reinterpret_cast<const T*>(P.q)[(int64_t)h0 * D + g * D + lane];
-  const int T_act = min(P.tokens_dev ? P.tokens_dev[0] + P.tokens : P.tokens, P.max_tokens);
-  if (c * kChunk >= T_act) return;
-  const bool valid = t < T_act;
-  const int nt = min(kChunk, T_act - c * kChunk);
-#pragma unroll
-  for (int g = 0; g < G; g++) q_s[g * D + lane] = to_f32(qraw[g]);
-  __syncthreads();
-  float sc[G];
-#pragma unroll
-  for (int g = 0; g < G; g++) sc[g] = 0.0f;
-#pragma unroll
-  for (int i = 0; i < D / 8; i++) {
-    const uint32_t kw[4] = {kr[i].x, kr[i].y, kr[i].z, kr[i].w};
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-      const float kv = (e & 1) ? hi_f32<T>(kw[e >> 1]) : lo_f32<T>(kw[e >> 1]);
-#pragma unroll
-      for (int g = 0; g < G; g++) sc[g] = __builtin_fmaf(q_s[g * D + 8 * i + e], kv, sc[g]);
-    }
-  }
-  const float ninf = __builtin_bit_cast(float, 0xff800000u);
-#pragma unroll
-  for (int g = 0; g < G; g++) {
-    const float s = valid ? sc[g] * P.scale : ninf;
-    float m = s;
-    m = fmaxf(m, xor_partner<1>(m));
-    m = fmaxf(m, xor_partner<2>(m));
-    m = fmaxf(m, xor_partner<4>(m));
-    m = fmaxf(m, xor_partner<8>(m));
-    m = fmaxf(m, xor_partner<16>(m));
-    m = fmaxf(m, xor_partner<32>(m));
-    const float p = valid ? exp_f32(s - m) : 0.0f;
-    const float l = xor_sum(p, 1, 64);
-    p_s[g * kChunk + lane] = p;
-    if (lane == 0) {
-      P.part_m[(int64_t)(h0 + g) * P.max_chunks + c] = m;
-      P.part_l[(int64_t)(h0 + g) * P.max_chunks + c] = l;
-    }
-  }
-  __syncthreads();
-  float o[G];
-#pragma unroll
-  for (int g = 0; g < G; g++) o[g] = 0.0f;
-#pragma unroll
-  for (int tt = 0; tt < kChunk; tt++) {
-    const float v = tt < nt ? to_f32(vraw[tt]) : 0.0f;
-#pragma unroll
-    for (int g = 0; g < G; g++) o[g] = __builtin_fmaf(p_s[g * kChunk + tt], v, o[g]);
-  }
-#pragma unroll
-  for (int g = 0; g < G; g++) P.part_o[((int64_t)(h0 + g) * P.max_chunks + c) * D + lane] = o[g];
-}
-
-// Combine of one head of dimension 64 (lane = dimension), the arithmetic of
-// combine_head; the chunk metadata and the partial outputs of up to kBlk chunks are
-// requested together before the maximum is formed.
-template <typename T, typename SKT>
-__global__ __launch_bounds__(64) void attn_combine64_kernel(AttnParams P) {
-  constexpr int D = 64, kBlk = 32;
-  const int h = blockIdx.x;
-  const int lane = threadIdx.x;
-  const int T_act = min(P.tokens_dev ? P.tokens_dev[0] + P.tokens : P.tokens, P.max_tokens);
-  const int nc = T_act > 0 ? (T_act + kChunk - 1) / kChunk : 0;
-  const float* pm = P.part_m + (int64_t)h * P.max_chunks;
-  const float* pl = P.part_l + (int64_t)h * P.max_chunks;
-  const float* po = P.part_o + (int64_t)h * P.max_chunks * D + lane;
-  const int last = P.max_chunks - 1;
-  // first block of every operand, clamped to the scratch (values past nc are unused)
-  float mv = pm[lane < last ? lane : last];
-  float lv = pl[lane < last ? lane : last];
-  float ov[kBlk];
-#pragma unroll
-  for (int u = 0; u < kBlk; u++) ov[u] = po[(int64_t)(u < last ? u : last) * D];
-  const float ninf = __builtin_bit_cast(float, 0xff800000u);
-  const bool has_sink = P.sinks != nullptr;
-  const float sink = has_sink ? to_f32(reinterpret_cast<const SKT*>(P.sinks)[h]) : 0.0f;
-  float M = has_sink ? sink : ninf;
-  for (int c0 = 0; c0 < nc; c0 += 64) {
-    float m = c0 + lane < nc ? (c0 == 0 ? mv : pm[c0 + lane]) : ninf;
-    m = fmaxf(m, xor_partner<1>(m));
-    m = fmaxf(m, xor_partner<2>(m));
-    m = fmaxf(m, xor_partner<4>(m));
-    m = fmaxf(m, xor_partner<8>(m));
-    m = fmaxf(m, xor_partner<16>(m));
-    m = fmaxf(m, xor_partner<32>(m));
-    M = fmaxf(M, m);
-  }
-  float den = has_sink ? exp_f32(sink - M) : 0.0f;
-  float acc = 0.0f;
-  for (int c0 = 0; c0 < nc; c0 += 64) {
-    const int n = min(64, nc - c0);
-    const float e = c0 + lane < nc ? exp_f32((c0 == 0 ? mv : pm[c0 + lane]) - M) : 0.0f;
-    const float l = c0 + lane < nc ? (c0 == 0 ? lv : pl[c0 + lane]) : 0.0f;
-    for (int c1 = 0; c1 < n; c1 += kBlk) {
-      if (c0 + c1 > 0) {
-#pragma unroll
-        for (int u = 0; u < kBlk; u++) {
-          const int cc = c0 + c1 + u;
-          ov[u] = po[(int64_t)(cc < last ? cc : last) * D];
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < kBlk; u++) {
-        if (c1 + u < n) {
-          const float ec = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, e), c1 + u));
-          const float lc = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, l), c1 + u));
-          den = __builtin_fmaf(lc, ec, den);
-          acc = __builtin_fmaf(ov[u], ec, acc);
-        }
-      }
-    }
-  }
-  store<T>(reinterpret_cast<T*>(P.out) + (int64_t)h * D + lane, acc / den);
-}
-
-// One workgroup per query head (contiguous head_dim-64 caches, whole-chunk capacity):
-// its kHeadWaves waves compute the head's chunk partials (chunk c on wave c mod
-// kHeadWaves) into LDS with the arithmetic of attn_partial64_kernel, and after one
-// barrier wave 0 combines them in chunk order with the arithmetic of
-// attn_combine64_kernel -- one launch, no communication between workgroups.
-//
-// Memory path: a wave requests its chunk's K and V blocks as sixteen fully coalesced
-// 16-byte loads per lane (each instruction covers 1 KB of consecutive bytes) and
-// transposes them through its own 8 KB LDS slice: K first (token r's piece d at slot
-// 8r + (d xor (r mod 8)), so the row reads of the score phase are free of bank
-// conflicts), then V in the same slice for the weighted sum.  The next chunk's blocks
-// are requested before the softmax so the value phase hides them.
-// Workgroups are dealt to the XCDs round-robin by id, so the query heads of one KV head
-// get ids congruent mod 8 (when the head counts allow it) and read its K/V rows through
-// one L2.
-constexpr int kHeadWaves = 12;
-constexpr int kHeadMaxChunks = 192;   // LDS partials: 66 floats per chunk
-constexpr int kXcds = 8;
-
-// A chunk's K and V blocks (64 tokens x 64 dims, 8 KB each) as 16-byte pieces
-// i * 64 + lane: token 8i + lane / 8, dimensions 8 (lane mod 8) .. +7.
-struct ChunkPieces {
-  uint4 k[8], v[8];
-};
-
-__device__ __forceinline__ ChunkPieces load_chunk(const uint4* kbase, const uint4* vbase, int c, int lane) {
-  const uint4* kblk = kbase + (int64_t)c * (kChunk * 64 / 8);
-  const uint4* vblk = vbase + (int64_t)c * (kChunk * 64 / 8);
-  ChunkPieces r;
-#pragma unroll
-  for (int i = 0; i < 8; i++) r.k[i] = kblk[i * 64 + lane];
-#pragma unroll
-  for (int i = 0; i < 8; i++) r.v[i] = vblk[i * 64 + lane];
-  return r;
-}
-
-template <typename T, typename SKT>
-__global__ __launch_bounds__(64 * kHeadWaves) void attn_head_kernel(AttnParams P) {
-  constexpr int D = 64;
-  const int G = P.heads / P.kv_heads;
-  int h = blockIdx.x;
-  if (P.heads % kXcds == 0 && P.kv_heads % kXcds == 0) {
-    // workgroup w runs on XCD w mod 8; its slot j = w / 8 on that XCD names
-    // (KV head 8 * (j / G) + w mod 8, query head j mod G of that group)
-    const int x = h % kXcds, j = h / kXcds;
-    h = ((j / G) * kXcds + x) * G + j % G;
-  }
-  const int kvh = h / G;
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  __shared__ float q_s[D];
-  __shared__ float p_s[kHeadWaves][kChunk];
-  __shared__ uint4 kv_s[kHeadWaves][kChunk * D / 8];
-  __shared__ float pm_s[kHeadMaxChunks], pl_s[kHeadMaxChunks];
-  __shared__ float po_s[kHeadMaxChunks][D];
-  const float ninf = __builtin_bit_cast(float, 0xff800000u);
-  const uint4* kbase = reinterpret_cast<const uint4*>(reinterpret_cast<const T*>(P.keys) + kvh * P.k_head);
-  const uint4* vbase = reinterpret_cast<const uint4*>(reinterpret_cast<const T*>(P.values) + kvh * P.v_head);
-  // first chunk of this wave: every load is issued before the active count is known
-  // (chunks below max_chunks are inside the capacity)
-  const int c_first = wave;
-  ChunkPieces cur;
-  if (c_first < P.max_chunks) cur = load_chunk(kbase, vbase, c_first, lane);
-  const T qraw = reinterpret_cast<const T*>(P.q)[(int64_t)h * D + lane];
-  const int T_act = min(P.tokens_dev ? P.tokens_dev[0] + P.tokens : P.tokens, P.max_tokens);
-  const int nc = T_act > 0 ? (T_act + kChunk - 1) / kChunk : 0;
-  if (wave == 0) q_s[lane] = to_f32(qraw);
-  __syncthreads();
-
-  float* p_w = p_s[wave];
-  uint4* kv_w = kv_s[wave];
-  for (int c = c_first; c < nc; c += kHeadWaves) {
-    const int t = c * kChunk + lane;
-    const bool valid = t < T_act;
-    const int nt = min(kChunk, T_act - c * kChunk);
-    // K block into the slice, then this lane's token row back out of it
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const int r = i * 8 + (lane >> 3);
-      const uint4 k = cur.k[i];
-      kv_w[r * 8 + ((lane & 7) ^ (r & 7))] = uint4{k.x, k.y, k.z, k.w};
-    }
-    __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): the K stores are done
-    __builtin_amdgcn_wave_barrier();
-    uint32_t krow[8][4];
-#pragma unroll
-    for (int d = 0; d < 8; d++) {
-      const uint4 k = kv_w[lane * 8 + (d ^ (lane & 7))];
-      krow[d][0] = k.x; krow[d][1] = k.y; krow[d][2] = k.z; krow[d][3] = k.w;
-    }
-    // V pieces of tokens past the count are staged as zeros: the weighted sum then adds
-    // fma(0, 0, o) == o for them (p is 0 there and o is never -0).  The wave's LDS
-    // operations complete in order, so these stores follow the row reads above.
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const uint32_t keep = i * 8 + (lane >> 3) < nt ? ~0u : 0u;
-      kv_w[i * 64 + lane] = uint4{cur.v[i].x & keep, cur.v[i].y & keep, cur.v[i].z & keep, cur.v[i].w & keep};
-    }
-    // score: fma chain over d ascending, lane = token
-    float sc = 0.0f;
-#pragma unroll
-    for (int i = 0; i < D / 8; i++) {
-      if ((i & 3) == 0) asm volatile("" : "+v"(sc)::"memory");   // 32 query values live per step
-      const uint32_t* kw = krow[i];
-#pragma unroll
-      for (int e = 0; e < 8; e++) {
-        const float kv = (e & 1) ? hi_f32<T>(kw[e >> 1]) : lo_f32<T>(kw[e >> 1]);
-        sc = __builtin_fmaf(q_s[8 * i + e], kv, sc);
-      }
-    }
-    // the next chunk of this wave is requested while this one finishes
-    if (c + kHeadWaves < nc) cur = load_chunk(kbase, vbase, c + kHeadWaves, lane);
-    const float s = valid ? sc * P.scale : ninf;
-    float m = s;
-    m = fmaxf(m, xor_partner<1>(m));
-    m = fmaxf(m, xor_partner<2>(m));
-    m = fmaxf(m, xor_partner<4>(m));
-    m = fmaxf(m, xor_partner<8>(m));
-    m = fmaxf(m, xor_partner<16>(m));
-    m = fmaxf(m, xor_partner<32>(m));
-    const float p = valid ? exp_f32(s - m) : 0.0f;
-    const float l = xor_sum(p, 1, 64);
-    p_w[lane] = p;
-    if (lane == 0) {
-      pm_s[c] = m;
-      pl_s[c] = l;
-    }
-    __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): this wave's p and V stores done
-    __builtin_amdgcn_wave_barrier();
-    // weighted values: lane = dimension, fma chain over the chunk's tokens ascending
-    const T* vs = reinterpret_cast<const T*>(kv_w);
-    float o = 0.0f;
-#pragma unroll
-    for (int tt = 0; tt < kChunk; tt++) {
-      if ((tt & 31) == 0) asm volatile("" : "+v"(o)::"memory");   // 32 tokens live per step
-      o = __builtin_fmaf(p_w[tt], to_f32(vs[tt * D + lane]), o);
-    }
-    po_s[c][lane] = o;
-    __builtin_amdgcn_s_waitcnt(0xc07f);   // reads of the wave's LDS slices done before reuse
-    __builtin_amdgcn_wave_barrier();
-  }
-  __syncthreads();
-  if (wave != 0) return;
-
-  // combine in chunk order (the arithmetic of combine_head)
-  const bool has_sink = P.sinks != nullptr;
-  const float sink = has_sink ? to_f32(reinterpret_cast<const SKT*>(P.sinks)[h]) : 0.0f;
-  float M = has_sink ? sink : ninf;
-  for (int c0 = 0; c0 < nc; c0 += 64) {
-    float mm = c0 + lane < nc ? pm_s[c0 + lane] : ninf;
-    mm = fmaxf(mm, xor_partner<1>(mm));
-    mm = fmaxf(mm, xor_partner<2>(mm));
-    mm = fmaxf(mm, xor_partner<4>(mm));
-    mm = fmaxf(mm, xor_partner<8>(mm));
-    mm = fmaxf(mm, xor_partner<16>(mm));
-    mm = fmaxf(mm, xor_partner<32>(mm));
-    M = fmaxf(M, mm);
-  }
-  float den = has_sink ? exp_f32(sink - M) : 0.0f;
-  float acc = 0.0f;
-  for (int c0 = 0; c0 < nc; c0 += 64) {
-    const int n = min(64, nc - c0);
-    const float e = c0 + lane < nc ? exp_f32(pm_s[c0 + lane] - M) : 0.0f;
-    const float lv = c0 + lane < nc ? pl_s[c0 + lane] : 0.0f;
-    for (int u = 0; u < n; u++) {
-      const float ec = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, e), u));
-      const float lc = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lv), u));
-      den = __builtin_fmaf(lc, ec, den);
-      acc = __builtin_fmaf(po_s[c0 + u][lane], ec, acc);
-    }
-  }
-  store<T>(reinterpret_cast<T*>(P.out) + (int64_t)h * D + lane, acc / den);
-}
-
 // One workgroup per (KV head, chunk) with one wave per query head of that KV head
 // (contiguous head_dim-64 caches, whole-chunk capacity): the chunk's K and V blocks are
 // read once per KV head -- each CU moves 16 KB instead of a whole sequence -- staged in
-// LDS (K swizzled as in attn_head_kernel, V rows of tokens past the count zeroed), and
+// LDS (K row r's piece d at slot 8r + (d xor r mod 8), V rows of tokens past the count zeroed), and
 // wave g computes the chunk partial of query head G kvh + g with the arithmetic of
-// attn_partial64_kernel.  The partials go to the scratch with device-scope atomic stores;
+// attn_chunk.  The partials go to the scratch with device-scope atomic stores;
 // the workgroup counts itself in its KV head's arrival counter once its stores have
 // completed, and the last of the head's active chunks combines every query head of the
-// KV head in chunk order (the arithmetic of attn_combine64_kernel, partials read with
+// KV head in chunk order (the arithmetic of combine_head, partials read with
 // device-scope atomic loads) and resets the counter to zero.  No workgroup waits for
-// another.  Same bits as attn_head_kernel.
+// another.
 __device__ __forceinline__ void st_dev(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ float ld_dev(const float* p) {
   return __hip_atomic_load(const_cast<float*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <typename T, typename SKT, int G, int CPW = 1, bool COMBINE = true>
+template <typename T, typename SKT, int G, bool COMBINE = true>
 __global__ __launch_bounds__(64 * G) void attn_kvchunk_kernel(AttnParams P, int* counters) {
-  // CPW chunks per workgroup (1 or 2): with 2, both chunks' K and V pieces are requested
-  // up front and the chunks are computed one after the other through the same LDS, which
-  // halves the grid when it is several generations of workgroups deep; every chunk's
-  // partial is computed exactly as with one chunk per workgroup
-  static_assert(CPW == 1 || CPW == 2, "one or two chunks per workgroup");
   constexpr int D = 64;
-  const int c0 = blockIdx.x * CPW, kvh = blockIdx.y;
+  const int c = blockIdx.x, kvh = blockIdx.y;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int h = kvh * G + wave;
@@ -582,51 +214,38 @@ __global__ __launch_bounds__(64 * G) void attn_kvchunk_kernel(AttnParams P, int*
   __shared__ float p_s[G][kChunk];
   __shared__ int last;
   const float ninf = __builtin_bit_cast(float, 0xff800000u);
-  // every load before the active count is known (chunks below max_chunks are inside
-  // the capacity; a second chunk past them is clamped to the last one, values unused):
-  // K and V pieces of the chunks, this wave's query row
+  // every load before the active count is known (chunks below max_chunks are inside the
+  // capacity): K and V pieces of the chunk, this wave's query row
   constexpr int kPer = kChunk * D / 8 / nthr;   // 16-byte pieces per thread
   // (native 4-vectors: arrays of the uint4 struct type are kept in scratch memory here)
   typedef uint32_t piece_t __attribute__((ext_vector_type(4)));
-  piece_t kr[kPer], vr[kPer], kr1[kPer], vr1[kPer];
-  auto load_chunk = [&](int c, piece_t (&kk)[kPer], piece_t (&vv)[kPer]) {
+  piece_t kr[kPer], vr[kPer];
+  {
     const piece_t* kblk = reinterpret_cast<const piece_t*>(reinterpret_cast<const T*>(P.keys) + kvh * P.k_head) +
                           (int64_t)c * (kChunk * D / 8);
     const piece_t* vblk = reinterpret_cast<const piece_t*>(reinterpret_cast<const T*>(P.values) + kvh * P.v_head) +
                           (int64_t)c * (kChunk * D / 8);
 #pragma unroll
     for (int j = 0; j < kPer; j++) {
-      kk[j] = kblk[(int)threadIdx.x + nthr * j];
-      vv[j] = vblk[(int)threadIdx.x + nthr * j];
+      kr[j] = kblk[(int)threadIdx.x + nthr * j];
+      vr[j] = vblk[(int)threadIdx.x + nthr * j];
     }
-  };
-  load_chunk(c0, kr, vr);
-  if constexpr (CPW == 2) load_chunk(c0 + 1 < P.max_chunks ? c0 + 1 : P.max_chunks - 1, kr1, vr1);
+  }
   const T qraw = reinterpret_cast<const T*>(P.q)[(int64_t)h * D + lane];
   const int T_act = min(P.tokens_dev ? P.tokens_dev[0] + P.tokens : P.tokens, P.max_tokens);
   const int nc = T_act > 0 ? (T_act + kChunk - 1) / kChunk : 0;
-  if (c0 >= nc) return;
-  const int done = min(CPW, nc - c0);   // active chunks of this workgroup
+  if (c >= nc) return;
   q_s[wave][lane] = to_f32(qraw);
-
-#pragma unroll
-  for (int cc = 0; cc < CPW; cc++) {
-    if (cc >= done) break;   // uniform
-    const int c = c0 + cc;
-    if (cc > 0) __syncthreads();   // the previous chunk's LDS reads are done
+  {
     const int nt = min(kChunk, T_act - c * kChunk);
-    auto stage = [&](const piece_t (&kk)[kPer], const piece_t (&vv)[kPer]) {
 #pragma unroll
-      for (int j = 0; j < kPer; j++) {
-        const int pidx = (int)threadIdx.x + nthr * j;
-        const int r = pidx >> 3, col = pidx & 7;
-        reinterpret_cast<piece_t*>(ks)[r * 8 + (col ^ (r & 7))] = kk[j];
-        const uint32_t keep = r < nt ? ~0u : 0u;
-        reinterpret_cast<piece_t*>(vs_s)[pidx] = vv[j] & keep;
-      }
-    };
-    if (cc == 0) stage(kr, vr);
-    else stage(kr1, vr1);
+    for (int j = 0; j < kPer; j++) {
+      const int pidx = (int)threadIdx.x + nthr * j;
+      const int r = pidx >> 3, col = pidx & 7;
+      reinterpret_cast<piece_t*>(ks)[r * 8 + (col ^ (r & 7))] = kr[j];
+      const uint32_t keep = r < nt ? ~0u : 0u;
+      reinterpret_cast<piece_t*>(vs_s)[pidx] = vr[j] & keep;
+    }
     __syncthreads();
 
     // ---- chunk partial of query head h (lane = token, then lane = dimension)
@@ -684,11 +303,11 @@ __global__ __launch_bounds__(64 * G) void attn_kvchunk_kernel(AttnParams P, int*
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   if (threadIdx.x == 0)
-    last = __hip_atomic_fetch_add(counters + kvh, done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nc - done;
+    last = __hip_atomic_fetch_add(counters + kvh, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nc - 1;
   __syncthreads();
   if (!last) return;
 
-  // ---- combine of query head h in chunk order (attn_combine64_kernel's arithmetic); the
+  // ---- combine of query head h in chunk order (combine_head's arithmetic); the
   // first 64 chunks' (m, l) and the first kBlk chunks' partial rows are requested together
   // with the sink, one round trip, before the maximum is formed
   constexpr int kBlk = 32;
@@ -746,24 +365,314 @@ __global__ __launch_bounds__(64 * G) void attn_kvchunk_kernel(AttnParams P, int*
   if (threadIdx.x == 0) __hip_atomic_store(counters + kvh, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Two chunks per workgroup once the one-chunk grid holds more workgroups than this.
-constexpr int64_t kAttnPairMinWorkgroups = 1024;
+// ---------------------------------------------------------------- matrix-core partials
+// Chunk partials of head_dim 64 or 128 on the binary32 matrix cores: v_mfma_f32_4x4x1
+// multiplies, in sixteen blocks, a column of four rows by a row of four columns and adds the
+// products with one rounding each (a fused multiply-add, subnormals included; checked
+// against fmaf chains), so instruction k of a sequence is step k of sixty-four fma chains
+// for each of four query heads:
+//   * scores: lane = token, operand B its K row's element k, operand A the four heads' q_k;
+//     accumulator register g is head g's chain over d ascending;
+//   * values: lane = dimension (head_dim 128: two per lane), B the token's V element, A the
+//     four heads' p of the token.
+// One wave computes four query heads of one (KV head, chunk) -- K and V elements are
+// converted once for the four -- and a workgroup all heads of the KV head: it requests K, V
+// and query rows before the active count is known, K staged in LDS (rows xor-swizzled) for
+// the scores while V arrives.  Rows past the capacity are read at its last row; V rows past
+// the count are staged as zeros (p is 0 there, and fma(0, 0, o) == o).  Any token stride:
+// caches of a whole number of chunks or not.
+//
+// Partials and fold against what ran before (microseconds a call, graph-timed, caches in
+// rotation): heads / KV heads x head_dim, tokens -- 64 / 8 x 64, 16385: 42.8 -> 22.9 (one
+// wave per query head and one workgroup per KV head folding 257 chunks); 512 / 64 x 64,
+// 1025: 16.7 -> 14.8; 40 / 10 x 128, 4001: 30.8 -> 14.7; 64 / 8 x 128, 32768: 148 -> 49.5
+// (2.7 TB/s; both scalar loads before).  Past a few thousand tokens the partials bound it:
+// about 16 us at 4112 waves, vector and LDS work of about 480 and 130 instructions a wave
+// and the latency of 2 x 64 dependent MFMAs rather than memory.
+typedef float acc4_t __attribute__((ext_vector_type(4)));
+constexpr int kCountFirstChunks = 64;
+
+template <typename T, int G, int D>
+__global__ __launch_bounds__(64 * ((G + 3) / 4)) void attn_mfma_kernel(AttnParams P) {
+  static_assert(D == 64 || D == 128, "one or two dimensions per lane");
+  constexpr int W = (G + 3) / 4;                // waves, four query heads each
+  constexpr int HW = G < 4 ? G : 4;
+  constexpr int NV = D / 64;                    // dimensions per lane
+  constexpr int kRow = D / 8;                   // 16-byte pieces per row
+  constexpr int kPer = kChunk * kRow / (64 * W);   // pieces per thread
+  typedef uint32_t quad_t __attribute__((ext_vector_type(4)));
+  __shared__ quad_t kvs[kChunk * kRow];         // the K block, then the V block
+  __shared__ __attribute__((aligned(16))) float q_s[W][HW][D];
+  __shared__ __attribute__((aligned(16))) float p_s[W][HW][kChunk];
+  const int c = blockIdx.x, kvh = blockIdx.y;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int h0 = kvh * G + 4 * wave;
+  const int row = (lane & 3) < HW ? (lane & 3) : HW - 1;   // head of this lane's A operand
+  const T* kbase = reinterpret_cast<const T*>(P.keys) + kvh * P.k_head;
+  const T* vbase = reinterpret_cast<const T*>(P.values) + kvh * P.v_head;
+  // a grid of many chunks may lie mostly past the count: there it is read before anything else
+  if (P.max_chunks > kCountFirstChunks &&
+      c * kChunk >= (P.tokens_dev ? P.tokens_dev[0] + P.tokens : P.tokens))
+    return;
+  quad_t kr[kPer], vr[kPer];
+#pragma unroll
+  for (int j = 0; j < kPer; j++) {
+    const int f = (int)threadIdx.x + 64 * W * j;
+    const int64_t t = min(c * kChunk + f / kRow, P.max_tokens - 1);
+    kr[j] = *reinterpret_cast<const quad_t*>(kbase + t * P.k_tok + 8 * (f % kRow));
+  }
+#pragma unroll
+  for (int j = 0; j < kPer; j++) {
+    const int f = (int)threadIdx.x + 64 * W * j;
+    const int64_t t = min(c * kChunk + f / kRow, P.max_tokens - 1);
+    vr[j] = *reinterpret_cast<const quad_t*>(vbase + t * P.v_tok + 8 * (f % kRow));
+  }
+  T qraw[HW][NV];
+#pragma unroll
+  for (int g = 0; g < HW; g++)
+#pragma unroll
+    for (int n = 0; n < NV; n++) qraw[g][n] = reinterpret_cast<const T*>(P.q)[(int64_t)(h0 + g) * D + 64 * n + lane];
+  const int T_act = min(P.tokens_dev ? P.tokens_dev[0] + P.tokens : P.tokens, P.max_tokens);
+  __builtin_amdgcn_sched_barrier(0);   // every load above is requested first
+  if (c * kChunk >= T_act) return;
+  const int t = c * kChunk + lane;
+  const bool valid = t < T_act;
+  const int nt = min(kChunk, T_act - c * kChunk);
+#pragma unroll
+  for (int j = 0; j < kPer; j++) {
+    const int f = (int)threadIdx.x + 64 * W * j;
+    const int r = f / kRow, col = f % kRow;
+    kvs[r * kRow + (col ^ (r & (kRow - 1)))] = kr[j];
+  }
+#pragma unroll
+  for (int g = 0; g < HW; g++)
+#pragma unroll
+    for (int n = 0; n < NV; n++) q_s[wave][g][64 * n + lane] = to_f32(qraw[g][n]);
+  lds_barrier();
+
+  acc4_t sc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int i = 0; i < kRow; i++) {
+    const quad_t k8 = kvs[lane * kRow + (i ^ (lane & (kRow - 1)))];
+    const acc4_t qa = *reinterpret_cast<const acc4_t*>(&q_s[wave][row][8 * i]);
+    const acc4_t qb = *reinterpret_cast<const acc4_t*>(&q_s[wave][row][8 * i + 4]);
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      const uint32_t kw = k8[e >> 1];
+      const float kv = (e & 1) ? hi_f32<T>(kw) : lo_f32<T>(kw);
+      sc = __builtin_amdgcn_mfma_f32_4x4x1f32(e < 4 ? qa[e & 3] : qb[e & 3], kv, sc, 0, 0, 0);
+    }
+  }
+  if constexpr (W > 1) lds_barrier();   // every wave has read its K rows
+  // V pieces of tokens past the count as zeros
+#pragma unroll
+  for (int j = 0; j < kPer; j++) {
+    const int f = (int)threadIdx.x + 64 * W * j;
+    const uint32_t keep = f / kRow < nt ? ~0u : 0u;
+    kvs[f] = vr[j] & keep;
+  }
+  const float ninf = __builtin_bit_cast(float, 0xff800000u);
+  float sv[HW], m[HW], l[HW];
+#pragma unroll
+  for (int g = 0; g < HW; g++) m[g] = sv[g] = valid ? sc[g] * P.scale : ninf;
+#pragma unroll
+  for (int g = 0; g < HW; g++) m[g] = fmaxf(m[g], xor_partner<1>(m[g]));
+#pragma unroll
+  for (int g = 0; g < HW; g++) m[g] = fmaxf(m[g], xor_partner<2>(m[g]));
+#pragma unroll
+  for (int g = 0; g < HW; g++) m[g] = fmaxf(m[g], xor_partner<4>(m[g]));
+#pragma unroll
+  for (int g = 0; g < HW; g++) m[g] = fmaxf(m[g], xor_partner<8>(m[g]));
+#pragma unroll
+  for (int g = 0; g < HW; g++) m[g] = fmaxf(m[g], xor_partner<16>(m[g]));
+#pragma unroll
+  for (int g = 0; g < HW; g++) m[g] = fmaxf(m[g], xor_partner<32>(m[g]));
+#pragma unroll
+  for (int g = 0; g < HW; g++) {
+    l[g] = valid ? exp_f32(sv[g] - m[g]) : 0.0f;
+    p_s[wave][g][lane] = l[g];
+  }
+  lds_barrier();   // p and V are staged
+  acc4_t o[NV];
+#pragma unroll
+  for (int n = 0; n < NV; n++) o[n] = (acc4_t){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int t4 = 0; t4 < kChunk / 4; t4++) {
+    const acc4_t pa = *reinterpret_cast<const acc4_t*>(&p_s[wave][row][4 * t4]);
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const int tt = 4 * t4 + e;
+      if constexpr (D == 64) {
+        const T v = reinterpret_cast<const T*>(kvs)[tt * D + lane];
+        o[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(pa[e], to_f32(v), o[0], 0, 0, 0);
+      } else {
+        const uint32_t w = reinterpret_cast<const uint32_t*>(kvs)[tt * 64 + lane];
+        o[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(pa[e], lo_f32<T>(w), o[0], 0, 0, 0);
+        o[NV - 1] = __builtin_amdgcn_mfma_f32_4x4x1f32(pa[e], hi_f32<T>(w), o[NV - 1], 0, 0, 0);
+      }
+    }
+  }
+#pragma unroll
+  for (int g = 0; g < HW; g++) l[g] = xor_sum(l[g], 1, 64);
+#pragma unroll
+  for (int g = 0; g < HW; g++) {
+    const int64_t slot = (int64_t)(h0 + g) * P.max_chunks + c;
+    if (lane == 0) {
+      P.part_m[slot] = m[g];
+      P.part_l[slot] = l[g];
+    }
+    if constexpr (D == 64) {
+      P.part_o[slot * D + lane] = o[0][g];
+    } else {
+      typedef float f2_t __attribute__((ext_vector_type(2)));
+      *reinterpret_cast<f2_t*>(P.part_o + slot * D + 2 * lane) = (f2_t){o[0][g], o[NV - 1][g]};
+    }
+  }
+}
+
+// Fold of the chunk partials in chunk order (the arithmetic of combine_head), one workgroup
+// per (head, 64 dimensions).  Blocks of kFoldBlk chunks: the four waves request the block's
+// rows together (16 bytes a thread and load), leave them with e_c = exp(m_c - M) and l_c in
+// LDS, wave 0 runs the chains of the 64 dimensions and wave 1 the denominator's.
+constexpr int kFoldBlk = 128;
+
+// acc = fma(v[u STEP], e[u], acc) for u = 0 .. n - 1 in order, the next sixteen operands read
+// from LDS while sixteen are consumed (reads past n stay inside the kFoldBlk entries).
+template <int STEP>
+__device__ __forceinline__ void chain_step(const float* v, const float* e, int n, float& acc) {
+  float ov[2][16];
+  acc4_t ev[2][4];
+  auto load = [&](auto bc, int u) __attribute__((always_inline)) {
+    constexpr int b = decltype(bc)::value;
+#pragma unroll
+    for (int k = 0; k < 4; k++) ev[b][k] = *reinterpret_cast<const acc4_t*>(e + u + 4 * k);
+#pragma unroll
+    for (int k = 0; k < 16; k++) ov[b][k] = v[(u + k) * STEP];
+  };
+  auto use = [&](auto bc) __attribute__((always_inline)) {
+    constexpr int b = decltype(bc)::value;
+#pragma unroll
+    for (int k = 0; k < 16; k++) acc = __builtin_fmaf(ov[b][k], ev[b][k >> 2][k & 3], acc);
+  };
+  const std::integral_constant<int, 0> b0{};
+  const std::integral_constant<int, 1> b1{};
+  int u = 0;
+  load(b0, 0);
+  for (; u + 32 <= n; u += 32) {
+    load(b1, u + 16);
+    use(b0);
+    load(b0, u + 32 < kFoldBlk ? u + 32 : 0);
+    use(b1);
+  }
+  if (u + 16 <= n) {
+    use(b0);
+    u += 16;
+  }
+  for (; u < n; u++) acc = __builtin_fmaf(v[u * STEP], e[u], acc);
+}
+
+template <typename T, typename SKT>
+__global__ __launch_bounds__(256) void attn_fold_kernel(AttnParams P) {
+  const int h = blockIdx.x, d0 = 64 * blockIdx.y, D = P.head_dim;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  __shared__ __attribute__((aligned(16))) float rows[2][kFoldBlk][64];
+  __shared__ __attribute__((aligned(16))) float e_s[2][kFoldBlk], l_s[2][kFoldBlk];
+  __shared__ float red[4], den;
+  const float* pm = P.part_m + (int64_t)h * P.max_chunks;
+  const float* pl = P.part_l + (int64_t)h * P.max_chunks;
+  const float* po = P.part_o + (int64_t)h * P.max_chunks * D + d0;
+  acc4_t rr[kFoldBlk / 16];
+  float mr = 0.0f, lr = 0.0f;
+  auto request = [&](int c0, int last) __attribute__((always_inline)) {
+    const int cm = min(c0 + (tid & (kFoldBlk - 1)), last);
+    mr = pm[cm];
+    lr = pl[cm];
+#pragma unroll
+    for (int u = 0; u < kFoldBlk / 16; u++) {
+      const int cc = min(c0 + 16 * u + (tid >> 4), last);
+      rr[u] = *reinterpret_cast<const acc4_t*>(po + (int64_t)cc * D + 4 * (tid & 15));
+    }
+  };
+  const float ninf = __builtin_bit_cast(float, 0xff800000u);
+  const bool has_sink = P.sinks != nullptr;
+  const float sink = has_sink ? to_f32(reinterpret_cast<const SKT*>(P.sinks)[h]) : 0.0f;
+  const int T_act = min(P.tokens_dev ? P.tokens_dev[0] + P.tokens : P.tokens, P.max_tokens);
+  const int nc = T_act > 0 ? (T_act + kChunk - 1) / kChunk : 0;
+  const int last = nc > 0 ? nc - 1 : 0;
+  request(0, last);
+  float mm = ninf;   // the maximum ignores NaN and does not depend on the order
+  for (int c = tid; c < nc; c += 256) mm = fmaxf(mm, pm[c]);
+  mm = fmaxf(mm, xor_partner<1>(mm));
+  mm = fmaxf(mm, xor_partner<2>(mm));
+  mm = fmaxf(mm, xor_partner<4>(mm));
+  mm = fmaxf(mm, xor_partner<8>(mm));
+  mm = fmaxf(mm, xor_partner<16>(mm));
+  mm = fmaxf(mm, xor_partner<32>(mm));
+  if (lane == 0) red[wave] = mm;
+  lds_barrier();
+  float M = has_sink ? sink : ninf;
+  M = fmaxf(fmaxf(M, fmaxf(red[0], red[1])), fmaxf(red[2], red[3]));
+  float acc = wave == 1 && has_sink ? exp_f32(sink - M) : 0.0f;   // wave 1: the denominator
+  int buf = 0;
+  for (int c0 = 0; c0 < nc; c0 += kFoldBlk, buf ^= 1) {
+    if (tid < kFoldBlk) {
+      e_s[buf][tid] = exp_f32(mr - M);
+      l_s[buf][tid] = lr;
+    }
+#pragma unroll
+    for (int u = 0; u < kFoldBlk / 16; u++)
+      *reinterpret_cast<acc4_t*>(&rows[buf][16 * u + (tid >> 4)][4 * (tid & 15)]) = rr[u];
+    if (c0 + kFoldBlk < nc) request(c0 + kFoldBlk, last);
+    lds_barrier();   // alternating buffers: one barrier per block
+    const int n = min(kFoldBlk, nc - c0);
+    if (wave == 0) chain_step<64>(&rows[buf][0][lane], &e_s[buf][0], n, acc);
+    else if (wave == 1) chain_step<1>(&l_s[buf][0], &e_s[buf][0], n, acc);
+  }
+  if (tid == 64) den = acc;
+  __syncthreads();
+  if (wave == 0) store<T>(reinterpret_cast<T*>(P.out) + (int64_t)h * D + d0 + lane, acc / den);
+}
+
+template <typename T>
+static int launch_fold(const AttnParams& P, int sink_dtype, hipStream_t st) {
+  const dim3 grid(P.heads, P.head_dim / 64);
+  switch (sink_dtype) {
+    case TT_BF16: hipLaunchKernelGGL((attn_fold_kernel<T, bf16_t>), grid, dim3(256), 0, st, P); break;
+    case TT_F32: hipLaunchKernelGGL((attn_fold_kernel<T, float>), grid, dim3(256), 0, st, P); break;
+    default: hipLaunchKernelGGL((attn_fold_kernel<T, f16_t>), grid, dim3(256), 0, st, P); break;
+  }
+  return check_launch("gqa_attention");
+}
+
+// Operands that attn_mfma_kernel reads as they are: 16-byte pieces of K and V rows.
+static bool mfma_operands(const AttnParams& P) {
+  return (P.head_dim == 64 || P.head_dim == 128) && aligned(P.keys, 16) && P.k_tok % 8 == 0 &&
+         P.k_head % 8 == 0 && aligned(P.values, 16) && P.v_tok % 8 == 0 && P.v_head % 8 == 0;
+}
+
+template <typename T, int G>
+static int launch_mfma_partials(const AttnParams& P, hipStream_t st) {
+  const dim3 grid((unsigned)P.max_chunks, (unsigned)P.kv_heads), block(64 * ((G + 3) / 4));
+  if (P.head_dim == 64) hipLaunchKernelGGL((attn_mfma_kernel<T, G, 64>), grid, block, 0, st, P);
+  else hipLaunchKernelGGL((attn_mfma_kernel<T, G, 128>), grid, block, 0, st, P);
+  return check_launch("gqa_attention");
+}
+
+// Grids that one launch serves better than partials and fold: at most one workgroup per CU
+// and 32 chunks, where the second launch costs more than the last workgroup's fold (one
+// launch against two: 32 / 8 heads, 513 tokens 6.3 against 8.4 us, 64 / 8, 1025 tokens 7.8
+// against 8.4; 64 KV heads of 17 chunks 16.7 against 14.8, 8 of 65 chunks 15.5 against 9.1).
+static bool one_launch_grid(const AttnParams& P) {
+  return P.max_chunks <= 32 && (int64_t)P.max_chunks * P.kv_heads <= 256;
+}
 
 template <typename T, int G>
 static int launch_attn(const AttnParams& P, int sink_dtype, bool contiguous64, int* counters, hipStream_t st) {
   if constexpr (G <= 8) {
-    if (contiguous64 && counters != nullptr) {
-      const dim3 block(64 * G);
-      if ((int64_t)P.max_chunks * P.kv_heads > kAttnPairMinWorkgroups) {
-        const dim3 grid((unsigned)((P.max_chunks + 1) / 2), (unsigned)P.kv_heads);
-        switch (sink_dtype) {
-          case TT_BF16: hipLaunchKernelGGL((attn_kvchunk_kernel<T, bf16_t, G, 2>), grid, block, 0, st, P, counters); break;
-          case TT_F32: hipLaunchKernelGGL((attn_kvchunk_kernel<T, float, G, 2>), grid, block, 0, st, P, counters); break;
-          default: hipLaunchKernelGGL((attn_kvchunk_kernel<T, f16_t, G, 2>), grid, block, 0, st, P, counters); break;
-        }
-        return check_launch("gqa_attention");
-      }
-      const dim3 grid((unsigned)P.max_chunks, (unsigned)P.kv_heads);
+    if (contiguous64 && counters != nullptr && one_launch_grid(P)) {
+      const dim3 block(64 * G), grid((unsigned)P.max_chunks, (unsigned)P.kv_heads);
       switch (sink_dtype) {
         case TT_BF16: hipLaunchKernelGGL((attn_kvchunk_kernel<T, bf16_t, G>), grid, block, 0, st, P, counters); break;
         case TT_F32: hipLaunchKernelGGL((attn_kvchunk_kernel<T, float, G>), grid, block, 0, st, P, counters); break;
@@ -772,29 +681,11 @@ static int launch_attn(const AttnParams& P, int sink_dtype, bool contiguous64, i
       return check_launch("gqa_attention");
     }
   }
-  if (contiguous64 && P.max_chunks <= kHeadMaxChunks) {
-    switch (sink_dtype) {
-      case TT_BF16: hipLaunchKernelGGL((attn_head_kernel<T, bf16_t>), dim3(P.heads), dim3(64 * kHeadWaves), 0, st, P); break;
-      case TT_F32: hipLaunchKernelGGL((attn_head_kernel<T, float>), dim3(P.heads), dim3(64 * kHeadWaves), 0, st, P); break;
-      default: hipLaunchKernelGGL((attn_head_kernel<T, f16_t>), dim3(P.heads), dim3(64 * kHeadWaves), 0, st, P); break;
-    }
-    return check_launch("gqa_attention");
+  if (mfma_operands(P)) {
+    const int rc = launch_mfma_partials<T, G>(P, st);
+    return rc ? rc : launch_fold<T>(P, sink_dtype, st);
   }
-  if (contiguous64) {
-    hipLaunchKernelGGL((attn_partial64_kernel<T, G>), dim3(P.max_chunks, P.kv_heads), dim3(64), 0, st, P);
-    int rc = check_launch("gqa_attention");
-    if (rc) return rc;
-    switch (sink_dtype) {
-      case TT_BF16: hipLaunchKernelGGL((attn_combine64_kernel<T, bf16_t>), dim3(P.heads), dim3(64), 0, st, P); break;
-      case TT_F32: hipLaunchKernelGGL((attn_combine64_kernel<T, float>), dim3(P.heads), dim3(64), 0, st, P); break;
-      default: hipLaunchKernelGGL((attn_combine64_kernel<T, f16_t>), dim3(P.heads), dim3(64), 0, st, P); break;
-    }
-    return check_launch("gqa_attention");
-  }
-  if (contiguous64)
-    hipLaunchKernelGGL((attn_partial_kernel<T, G, 64>), dim3(P.max_chunks, P.kv_heads), dim3(64), 0, st, P);
-  else
-    hipLaunchKernelGGL((attn_partial_kernel<T, G, 0>), dim3(P.max_chunks, P.kv_heads), dim3(64), 0, st, P);
+  hipLaunchKernelGGL((attn_partial_kernel<T, G>), dim3(P.max_chunks, P.kv_heads), dim3(64), 0, st, P);
   int rc = check_launch("gqa_attention");
   if (rc) return rc;
   switch (sink_dtype) {
@@ -820,13 +711,9 @@ extern "C" int tt_attention_scratch_floats(int64_t heads, int64_t max_tokens, in
 // combines the partials itself (tt_attention_combine_int4_matvec).
 template <typename T, int G>
 static int launch_attn_partials(const AttnParams& P, hipStream_t st) {
-  const dim3 block(64 * G);
-  if ((int64_t)P.max_chunks * P.kv_heads > kAttnPairMinWorkgroups)
-    hipLaunchKernelGGL((attn_kvchunk_kernel<T, f16_t, G, 2, false>), dim3((unsigned)((P.max_chunks + 1) / 2), (unsigned)P.kv_heads),
-                       block, 0, st, P, nullptr);
-  else
-    hipLaunchKernelGGL((attn_kvchunk_kernel<T, f16_t, G, 1, false>), dim3((unsigned)P.max_chunks, (unsigned)P.kv_heads), block,
-                       0, st, P, nullptr);
+  if (!one_launch_grid(P)) return launch_mfma_partials<T, G>(P, st);
+  hipLaunchKernelGGL((attn_kvchunk_kernel<T, f16_t, G, false>), dim3((unsigned)P.max_chunks, (unsigned)P.kv_heads),
+                     dim3(64 * G), 0, st, P, nullptr);
   return check_launch("gqa_attention_partials");
 }
 
@@ -911,7 +798,7 @@ extern "C" int tt_single_token_gqa_attention(const void* q, const void* keys, co
   // 128-bit K loads and whole-chunk V loads need contiguous 64-wide rows and a
   // capacity that is a whole number of chunks
   const bool c64 = head_dim == 64 && k_tok == 64 && v_tok == 64 && max_tokens % kChunk == 0 && aligned(keys, 16) &&
-                   k_head % 8 == 0 && v_head % 8 == 0 && heads / kv_heads <= 8;
+                   aligned(values, 16) && k_head % 8 == 0 && v_head % 8 == 0 && heads / kv_heads <= 8;
   auto by_g = [&](auto t) -> int {
     using T = decltype(t);
     switch (G) {
