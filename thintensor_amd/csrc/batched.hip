@@ -610,6 +610,7 @@ int launch_mfma(MfmaParams P, hipStream_t st, const char* what) {
   int rc;
   if (mt == 1) rc = launch_mfma_mt<W, 1>(P, plan.nt, grid, st);
   else if (mt == 2) rc = launch_mfma_mt<W, 2>(P, plan.nt, grid, st);
+  else if (mt == 3) rc = launch_mfma_mt<W, 3>(P, plan.nt, grid, st);
   else rc = launch_mfma_mt<W, 4>(P, plan.nt, grid, st);
   return rc ? rc : check_launch(what);
 }
