@@ -19,6 +19,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("heads,kv_heads,dim,tokens,cap,bf16,sinks,pad", [
     (40, 10, 128, 130, 200, True, False, 0),     # four heads per KV head, capacity inside a chunk
     (2, 2, 128, 1, 1, False, True, 0),           # one head, one token, one-row cache
+    (1, 1, 128, 130, 130, False, False, 0),      # three chunk rows: partials off a 16-byte boundary
     (6, 3, 128, 64, 64, True, True, 0),          # two heads, exactly one chunk
     (8, 1, 64, 8257, 8300, False, True, 0),      # 130 chunks: a second fold block of two
     (16, 1, 64, 2050, 2050, False, False, 0),    # sixteen heads, four waves

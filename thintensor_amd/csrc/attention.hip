@@ -525,7 +525,7 @@ __global__ __launch_bounds__(64 * ((G + 3) / 4)) void attn_mfma_kernel(AttnParam
     if constexpr (D == 64) {
       P.part_o[slot * D + lane] = o[0][g];
     } else {
-      typedef float f2_t __attribute__((ext_vector_type(2)));
+      typedef float f2_t __attribute__((ext_vector_type(2), aligned(4)));
       *reinterpret_cast<f2_t*>(P.part_o + slot * D + 2 * lane) = (f2_t){o[0][g], o[NV - 1][g]};
     }
   }
@@ -583,6 +583,8 @@ __global__ __launch_bounds__(256) void attn_fold_kernel(AttnParams P) {
   const float* pm = P.part_m + (int64_t)h * P.max_chunks;
   const float* pl = P.part_l + (int64_t)h * P.max_chunks;
   const float* po = P.part_o + (int64_t)h * P.max_chunks * D + d0;
+  // the scratch's rows start at any multiple of eight bytes (2 heads max_chunks floats precede them)
+  typedef acc4_t row4_t __attribute__((aligned(4)));
   acc4_t rr[kFoldBlk / 16];
   float mr = 0.0f, lr = 0.0f;
   auto request = [&](int c0, int last) __attribute__((always_inline)) {
@@ -592,7 +594,7 @@ __global__ __launch_bounds__(256) void attn_fold_kernel(AttnParams P) {
 #pragma unroll
     for (int u = 0; u < kFoldBlk / 16; u++) {
       const int cc = min(c0 + 16 * u + (tid >> 4), last);
-      rr[u] = *reinterpret_cast<const acc4_t*>(po + (int64_t)cc * D + 4 * (tid & 15));
+      rr[u] = *reinterpret_cast<const row4_t*>(po + (int64_t)cc * D + 4 * (tid & 15));
     }
   };
   const float ninf = __builtin_bit_cast(float, 0xff800000u);
