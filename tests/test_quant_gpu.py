@@ -19,6 +19,7 @@ import pytest
 import torch
 
 from oracle import quant as Q
+from tests.helpers import rng
 from thintensor_amd import quantize as TQ
 
 pytestmark = pytest.mark.gpu
@@ -332,3 +333,24 @@ def test_int4_symmetric_edges(affine_env, mode, dtype, rows, cols, group):
     eq(got[0], as_np(want[0]), "codes with infinities")
     eq(got[1].view(torch.int16 if mode == "lsq" else torch.int32), as_np(want[1].view(torch.int16 if mode == "lsq" else torch.int32)),
        "scales with infinities")
+
+
+@pytest.mark.parametrize("mode", ["lsq", "rows"])
+def test_int4_symmetric_scale_significands(affine_env, mode):
+    """binary32 elements up to two ulps from the ties of their group's scale, whose significands
+    include all ones (divided), one and their neighbours, at small, ordinary and huge exponents."""
+    affine_env(False)
+    g = rng(41)
+    sig = np.concatenate([[0x800000, 0x800001, 0xfffffe, 0xffffff], g.integers(0x800000, 0x1000000, 252)])
+    s = sig.astype(np.float32) * np.float32(2.0) ** g.choice([-60, -25, 0, 90], 256).astype(np.float32)
+    h = g.choice(np.arange(1, 14, 2), (256, 64)) * 0.5 * g.choice([-1, 1], (256, 64))
+    x = (h * s[:, None].astype(np.float64)).astype(np.float32)
+    x = (x.view(np.int32) + g.integers(-2, 3, x.shape).astype(np.int32)).view(np.float32)
+    x[:, 0] = (7 * s.astype(np.float64)).astype(np.float32)
+    assert (x[3, 0] / np.float32(7) == s[3])     # the scale has the significand meant
+    call, oracle_of = (TQ.quantize_to_int4_cpu, Q.int4_lsq) if mode == "lsq" else (TQ.quantize_int4_rows, Q.int4_rows)
+    with np.errstate(over="ignore"):             # fp16 scales past 65504
+        want = oracle_of(x, 64)
+    got = call(torch.from_numpy(x).cuda(), group_size=64)
+    eq(got[0], want[0], "codes")
+    eq(got[1], want[1].view(np.uint16) if mode == "lsq" else want[1], "scales")

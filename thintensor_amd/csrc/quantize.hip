@@ -143,49 +143,60 @@ struct Q4Params {
 // grid is small: 512 x 1024 fp16 5.0 us with four, 2.8 with one; one wave per
 // group 3.7).
 //
-// The sums need no particular order here.  A nonzero code means |x| >= amax / 14, so every
-// nonzero product x q lies within 2^4 of the largest x: with 24-bit products the sum over 512
-// elements spans at most 9 + 3 + 4 + 24 = 40 bits and is exact in binary64, and with 11-bit
-// sources the sum over a lane's eight elements spans 3 + 3 + 5 + 10 = 21 bits and is exact in
-// binary32.  (NaN and infinite elements give NaN in every order.)
+// The sums need no particular order here.  A nonzero code means |x| >= amax / 14, so with
+// 2^e <= amax < 2^(e + 1) every nonzero product x q is a multiple of 2^(e - 4 - p) for sources
+// of p + 1 significant bits and the sum over n elements is below 2^(e + 4) n: exact in binary64
+// for n = 512 binary32 sources (p = 23), in binary32 for n = 64 fp16 ones (p = 10: eight lanes)
+// and n = 512 bf16 ones (p = 7).  (NaN and infinite elements give NaN in every order; the
+// products are not negative, so a sum past the largest binary32 number is infinite in every
+// order.)
 //
-// rint(x / s) is taken from x * rcp(s) unless that lies within 1e-5 of a half-integer (or is
-// not finite): product (rcp is good to one ulp below 2^126, where its result is normal) and
-// quotient are both within 3e-6 of the true value while it is below 9, past which both clamp
-// alike.  A lane that is closer divides, its wave with it (bf16 sources often: x / amax is
-// then an odd multiple of 1 / 14 for some x of every seventh amax).
+// rint(x / s) is rint of a product with the reciprocal and one residual step, five operations
+// of one rounding each.  Its value next to every half-integer up to 8.5 equals that of the
+// quotient for every 24-bit significand of s but all ones and every reciprocal within an ulp of
+// 1 / s (all of them tried, x up to four ulps from the tie); elsewhere the step is within an ulp
+// of the quotient and past 8.5 both clamp alike.  Groups where a step could overflow or the
+// reciprocal is not normal, and that one significand, divide.
 //
-// Bound by HBM and the vector units about equally.  17920 x 5120 bf16, group 128: one wave
-// per group with binary64 folds over 64 lanes and two divisions per element 280 -> 89 us on
-// fresh buffers (2.6 TB/s; fp16 74 us, fp32 250 -> 82 us; group 32, half of whose waves'
-// lanes idled, fp16 855 -> 60 us).
+// Bound by the vector units for 16-bit sources, by HBM for binary32.  17920 x 5120, group 128,
+// graph of calls over four sources: bf16 288 us with one wave per group, binary64 folds over 64
+// lanes and two divisions per element; 82 with eight elements per lane and divisions in lanes
+// near a tie (often: x / amax is an odd multiple of 1 / 14 for some x of every seventh amax);
+// 61 as here (3.8 TB/s).  fp16 283, 69, 64; fp32 260, 81, 81 (5.1 TB/s); group 32, half of whose
+// waves' lanes idled, bf16 857, 80, 59.  2048 x 2048: bf16 15.6, 7.8, 6.9; fp32, whose elements
+// are seldom near a tie, 15.6, 7.7, 8.3.
 constexpr int kQ4Pieces = 4;
 
-template <int GL, typename T, typename F>
+// Steps FROM, 2 FROM, ... GL / 2 of the fold over GL lanes.
+template <int GL, int FROM = 1, typename T, typename F>
 __device__ __forceinline__ T fold_lanes(T v, F&& op) {
-  if constexpr (GL > 1) v = op(v, std::integral_constant<int, 1>{});
-  if constexpr (GL > 2) v = op(v, std::integral_constant<int, 2>{});
-  if constexpr (GL > 4) v = op(v, std::integral_constant<int, 4>{});
-  if constexpr (GL > 8) v = op(v, std::integral_constant<int, 8>{});
-  if constexpr (GL > 16) v = op(v, std::integral_constant<int, 16>{});
-  if constexpr (GL > 32) v = op(v, std::integral_constant<int, 32>{});
+  if constexpr (GL > 1 && FROM <= 1) v = op(v, std::integral_constant<int, 1>{});
+  if constexpr (GL > 2 && FROM <= 2) v = op(v, std::integral_constant<int, 2>{});
+  if constexpr (GL > 4 && FROM <= 4) v = op(v, std::integral_constant<int, 4>{});
+  if constexpr (GL > 8 && FROM <= 8) v = op(v, std::integral_constant<int, 8>{});
+  if constexpr (GL > 16 && FROM <= 16) v = op(v, std::integral_constant<int, 16>{});
+  if constexpr (GL > 32 && FROM <= 32) v = op(v, std::integral_constant<int, 32>{});
   return v;
 }
 
-// rint(x / s), clamped to [lo, 7] with CLAMP.  NaN and infinite quotients come out alike on
-// both paths, so the maximum may skip their NaN distances.
+// Lanes whose products' sum is exact in binary32 (the comment above).
+template <typename ST> constexpr int kExactLanes = 1;
+template <> constexpr int kExactLanes<f16_t> = 8;
+template <> constexpr int kExactLanes<bf16_t> = 64;
+
+// rint(x / s), clamped to [lo, 7] with CLAMP; amax the group's largest |x| that is not NaN.
 template <bool CLAMP>
-__device__ __forceinline__ void round_codes(const float (&x)[8], float s, float lo, float (&q)[8]) {
-  const float r = __builtin_amdgcn_rcpf(s);
-  float far = 0.0f;   // largest distance of a product from its nearest integer
+__device__ __forceinline__ void round_codes(const float (&x)[8], float amax, float s, float lo, float (&q)[8]) {
+  const float r0 = __builtin_amdgcn_rcpf(s);
+  const float r = __builtin_fmaf(__builtin_fmaf(-s, r0, 1.0f), r0, r0);
+  if (amax * r < 0x1p20f && s < 0x1p126f && (__builtin_bit_cast(uint32_t, s) & 0x7fffffu) != 0x7fffffu) {
 #pragma unroll
-  for (int k = 0; k < 8; k++) {
-    const float t = x[k] * r;
-    const float n = __builtin_rintf(t);
-    far = fmaxf(far, fabsf(t - n));
-    q[k] = CLAMP ? clampf(n, lo, 7.0f) : n;
-  }
-  if (far > 0.49999f || !(s < 0x1p126f)) {
+    for (int k = 0; k < 8; k++) {
+      const float t = x[k] * r;
+      const float n = __builtin_rintf(__builtin_fmaf(__builtin_fmaf(-t, s, x[k]), r, t));
+      q[k] = CLAMP ? clampf(n, lo, 7.0f) : n;
+    }
+  } else {
 #pragma unroll
     for (int k = 0; k < 8; k++) {
       const float n = __builtin_rintf(x[k] / s);
@@ -244,11 +255,11 @@ __global__ __launch_bounds__(256) void int4_sym_kernel(const Q4Params P, int ppr
     float s = fmaxf(amax, kTiny) / 7.0f;
     float q[8];
     if constexpr (!LSQ) {
-      round_codes<true>(x, s, -7.0f, q);
+      round_codes<true>(x, amax, s, -7.0f, q);
     } else {
       // |x / s| <= 7 unless x is NaN or infinite; a NaN product makes the sum NaN whatever its
       // code, an infinite one only with the clamped code
-      round_codes<false>(x, s, 0.0f, q);
+      round_codes<false>(x, amax, s, 0.0f, q);
       if (amax == __builtin_inff()) {
 #pragma unroll
         for (int k = 0; k < 8; k++) q[k] = clampf(q[k], -8.0f, 7.0f);
@@ -262,14 +273,15 @@ __global__ __launch_bounds__(256) void int4_sym_kernel(const Q4Params P, int ppr
         float part = 0.0f;
 #pragma unroll
         for (int k = 0; k < 8; k++) part = __builtin_fmaf(x[k], q[k], part);
-        num = (double)part;
+        constexpr int kLanes = GL < kExactLanes<ST> ? GL : kExactLanes<ST>;
+        num = (double)fold_lanes<kLanes>(part, [](float v, auto m) { return v + xor_partner<decltype(m)::value>(v); });
       }
 #pragma unroll
       for (int k = 0; k < 8; k++) den = __builtin_fmaf(q[k], q[k], den);
-      num = fold_lanes<GL>(num, [](double v, auto m) { return v + xor_partner_d<decltype(m)::value>(v); });
+      num = fold_lanes<GL, kExactLanes<ST>>(num, [](double v, auto m) { return v + xor_partner_d<decltype(m)::value>(v); });
       den = fold_lanes<GL>(den, [](float v, auto m) { return v + xor_partner<decltype(m)::value>(v); });
       s = fmaxf(fabsf((float)num / fmaxf(den, 1.0f)), kTiny);
-      round_codes<true>(x, s, -8.0f, q);
+      round_codes<true>(x, amax, s, -8.0f, q);
     }
     // four codes + 8 as one exact binary32 number
     const float lo4 = __builtin_fmaf(4096.0f, q[3], __builtin_fmaf(256.0f, q[2], __builtin_fmaf(16.0f, q[1], q[0]))) + 34952.0f;
