@@ -354,3 +354,15 @@ def test_int4_symmetric_scale_significands(affine_env, mode):
     got = call(torch.from_numpy(x).cuda(), group_size=64)
     eq(got[0], want[0], "codes")
     eq(got[1], want[1].view(np.uint16) if mode == "lsq" else want[1], "scales")
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_int4_symmetric_pieces_per_thread(affine_env, dtype):
+    """Large 16-bit matrices take several pieces per thread: the same codes and scales as
+    their row blocks, which take one (compared with the oracle above)."""
+    affine_env(False)
+    w = (torch.randn((8197, 2056), generator=torch.Generator().manual_seed(5)) * 0.02).to(dtype).cuda()
+    got = TQ.quantize_to_int4_cpu(w, group_size=64)
+    parts = [TQ.quantize_to_int4_cpu(w[r:r + 1000], group_size=64) for r in range(0, len(w), 1000)]
+    assert torch.equal(got[0], torch.cat([p[0] for p in parts]))
+    assert torch.equal(got[1], torch.cat([p[1] for p in parts]))

@@ -139,9 +139,8 @@ struct Q4Params {
 
 // Symmetric INT4 (kLsq, kRows) for widths that are a multiple of eight and 16-byte aligned
 // rows: eight consecutive elements per lane, GL = G / 8 lanes per group, 64 / GL groups per
-// wave, up to kQ4Pieces pieces per thread requested before the first is used (one while the
-// grid is small: 512 x 1024 fp16 5.0 us with four, 2.8 with one; one wave per
-// group 3.7).
+// wave, one or kQ4Pieces pieces per thread, all requested before the first is used (the rule
+// and its figures stand at the launch).
 //
 // The sums need no particular order here.  A nonzero code means |x| >= amax / 14, so with
 // 2^e <= amax < 2^(e + 1) every nonzero product x q is a multiple of 2^(e - 4 - p) for sources
@@ -162,9 +161,9 @@ struct Q4Params {
 // graph of calls over four sources: bf16 288 us with one wave per group, binary64 folds over 64
 // lanes and two divisions per element; 82 with eight elements per lane and divisions in lanes
 // near a tie (often: x / amax is an odd multiple of 1 / 14 for some x of every seventh amax);
-// 61 as here (3.8 TB/s).  fp16 283, 69, 64; fp32 260, 81, 81 (5.1 TB/s); group 32, half of whose
-// waves' lanes idled, bf16 857, 80, 59.  2048 x 2048: bf16 15.6, 7.8, 6.9; fp32, whose elements
-// are seldom near a tie, 15.6, 7.7, 8.3.
+// 61 as here (3.8 TB/s).  fp16 283, 69, 64; fp32 260, 81, 79 (5.2 TB/s); group 32, half of whose
+// waves' lanes idled, bf16 857, 80, 59.  2048 x 2048: bf16 15.6, 7.8, 5.6; fp32 15.6,
+// 7.7, 6.7.
 constexpr int kQ4Pieces = 4;
 
 // Steps FROM, 2 FROM, ... GL / 2 of the fold over GL lanes.
@@ -823,8 +822,14 @@ extern "C" int tt_quantize_int4(const void* src, int src_dtype, int64_t rows, in
           else hipLaunchKernelGGL((int4_sym_kernel<ST, GL, false, NP>), grid, dim3(256), 0, st, P, (int)ppr);
           return check_launch(what);
         };
-        if (pieces < 256 * 2048) return launch(std::integral_constant<int, 1>{});
-        return launch(std::integral_constant<int, kQ4Pieces>{});
+        // four pieces per thread pay for 16-bit sources of large matrices: 17920 x 5120 bf16 68 us
+        // with one, 62 with two or eight, 60 with four; 5000 x 4096 18.1, 17.7 (two), 18.4 (four);
+        // 2048 x 2048 5.6 against 6.9.  binary32 sources, two loads a piece: 77 - 80 us against
+        // 81 - 84, 20.4 against 21.9, 6.7 against 8.4
+        if constexpr (sizeof(ST) == 2) {
+          if (pieces >= 256 * 8192) return launch(std::integral_constant<int, kQ4Pieces>{});
+        }
+        return launch(std::integral_constant<int, 1>{});
       };
       switch (group_size) {
         case 32: return go(std::integral_constant<int, 4>{});
