@@ -413,7 +413,10 @@ int tt_attention_scratch_floats(int64_t heads, int64_t max_tokens, int64_t head_
 /* Single-token GQA attention over keys/values [kv_heads, tokens, D] (strides in
  * elements) with optional sinks [heads]; the token count is `tokens`, or
  * tokens_dev[0] + tokens when tokens_dev (int32) is non-null (a decode step passes its
- * position and 1).  max_tokens bounds the count (it sizes the scratch).  out [heads, D].
+ * position and 1).  max_tokens bounds the count and sizes the scratch.  Contiguous
+ * head_dim-64 caches of a whole number of 64-token chunks are requested before the count is
+ * known and must hold max_tokens rows; of any other cache only rows below the count are
+ * read.  out [heads, D].
  * Replaces TritonDecodeBackend.single_token_gqa_attention and
  * split_single_token_gqa_attention (triton_kernels.py:5228-5363; kernels :15-245). */
 int tt_single_token_gqa_attention(const void* q, const void* keys, const void* values, int dtype,

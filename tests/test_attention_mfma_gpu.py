@@ -10,8 +10,9 @@ import pytest
 import torch
 
 import oracle
-from tests.helpers import rng, to_torch
+from tests.helpers import f16_normal, from_torch_bits, rng, to_torch
 from tests.test_gemv_gpu import assert_bits_equal
+from thintensor_amd import _lib
 
 pytestmark = pytest.mark.gpu
 
@@ -56,3 +57,30 @@ def test_attention_partials_and_fold(backend, device, heads, kv_heads, dim, toke
                                    sk.ctypes.data if sinks else None, code, n, heads, kv_heads, dim, want.ctypes.data)
         got = out.cpu().view(torch.int16).numpy().view(np.uint16)
         assert_bits_equal(got, want.view(np.uint16), f"{n} tokens")
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,tokens,max_tokens", [(8, 2, 128, 130, 1000), (40, 10, 128, 64, 4500),
+                                                                  (8, 8, 64, 77, 200)])
+def test_rows_past_the_count_need_not_exist(backend, device, heads, kv_heads, dim, tokens, max_tokens):
+    """max_tokens bounds the count and sizes the scratch; caches that are not contiguous
+    head_dim-64 rows of whole chunks are read below the count only.  Here the last KV head
+    ends with the tensor, `tokens` rows long, so a read past the count leaves the
+    allocation."""
+    g = rng(heads + dim)
+    q, keys, vals = (f16_normal(g, s) for s in ((heads * dim,), (kv_heads, tokens, dim), (kv_heads, tokens, dim)))
+    qd, kd, vd = (to_torch(a, device) for a in (q, keys, vals))
+    out = torch.empty(heads * dim, device=device, dtype=torch.float16)
+    floats = backend.lib.tt_attention_scratch_floats(heads, max_tokens, dim)
+    scratch = torch.zeros(floats, device=device)
+    count = torch.tensor([tokens], dtype=torch.int32, device=device)
+    want = np.empty(heads * dim, dtype=np.float16)
+    oracle.lib().tto_attention(q.ctypes.data, keys.ctypes.data, vals.ctypes.data, oracle.F16, tokens * dim, dim,
+                               tokens * dim, dim, None, oracle.F16, tokens, heads, kv_heads, dim, want.ctypes.data)
+    for dev, n in ((None, tokens), (count.data_ptr(), 0)):
+        out.fill_(7.0)
+        rc = backend.lib.tt_single_token_gqa_attention(
+            qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), _lib.F16, tokens * dim, dim, tokens * dim, dim, None, _lib.F16,
+            dev, n, max_tokens, heads, kv_heads, dim, scratch.data_ptr(), floats, out.data_ptr(),
+            torch.cuda.current_stream(device).cuda_stream)
+        _lib.check(rc, "single_token_gqa_attention")
+        assert_bits_equal(from_torch_bits(out), want, "device count" if dev else "host count")

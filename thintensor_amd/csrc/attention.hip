@@ -376,11 +376,12 @@ __global__ __launch_bounds__(64 * G) void attn_kvchunk_kernel(AttnParams P, int*
 //   * values: lane = dimension (head_dim 128: two per lane), B the token's V element, A the
 //     four heads' p of the token.
 // One wave computes four query heads of one (KV head, chunk) -- K and V elements are
-// converted once for the four -- and a workgroup all heads of the KV head: it requests K, V
-// and query rows before the active count is known, K staged in LDS (rows xor-swizzled) for
-// the scores while V arrives.  Rows past the capacity are read at its last row; V rows past
-// the count are staged as zeros (p is 0 there, and fma(0, 0, o) == o).  Any token stride:
-// caches of a whole number of chunks or not.
+// converted once for the four -- and a workgroup all heads of the KV head: it reads the active
+// count, then requests K, V and query rows together, K staged in LDS (rows xor-swizzled) for
+// the scores while V arrives.  Only rows below the count are read (a caller's cache need not
+// hold max_tokens rows); rows past it repeat the last one and are staged as zeros for V (p is
+// 0 there, and fma(0, 0, o) == o).  Any token stride: caches of a whole number of chunks or
+// not.
 //
 // Partials and fold against what ran before (microseconds a call, graph-timed, caches in
 // rotation): heads / KV heads x head_dim, tokens -- 64 / 8 x 64, 16385: 42.8 -> 22.9 (one
@@ -390,7 +391,6 @@ __global__ __launch_bounds__(64 * G) void attn_kvchunk_kernel(AttnParams P, int*
 // about 16 us at 4112 waves, vector and LDS work of about 480 and 130 instructions a wave
 // and the latency of 2 x 64 dependent MFMAs rather than memory.
 typedef float acc4_t __attribute__((ext_vector_type(4)));
-constexpr int kCountFirstChunks = 64;
 
 template <typename T, int G, int D>
 __global__ __launch_bounds__(64 * ((G + 3) / 4)) void attn_mfma_kernel(AttnParams P) {
@@ -411,21 +411,19 @@ __global__ __launch_bounds__(64 * ((G + 3) / 4)) void attn_mfma_kernel(AttnParam
   const int row = (lane & 3) < HW ? (lane & 3) : HW - 1;   // head of this lane's A operand
   const T* kbase = reinterpret_cast<const T*>(P.keys) + kvh * P.k_head;
   const T* vbase = reinterpret_cast<const T*>(P.values) + kvh * P.v_head;
-  // a grid of many chunks may lie mostly past the count: there it is read before anything else
-  if (P.max_chunks > kCountFirstChunks &&
-      c * kChunk >= (P.tokens_dev ? P.tokens_dev[0] + P.tokens : P.tokens))
-    return;
+  const int T_act = min(P.tokens_dev ? P.tokens_dev[0] + P.tokens : P.tokens, P.max_tokens);
+  if (c * kChunk >= T_act) return;
   quad_t kr[kPer], vr[kPer];
 #pragma unroll
   for (int j = 0; j < kPer; j++) {
     const int f = (int)threadIdx.x + 64 * W * j;
-    const int64_t t = min(c * kChunk + f / kRow, P.max_tokens - 1);
+    const int64_t t = min(c * kChunk + f / kRow, T_act - 1);
     kr[j] = *reinterpret_cast<const quad_t*>(kbase + t * P.k_tok + 8 * (f % kRow));
   }
 #pragma unroll
   for (int j = 0; j < kPer; j++) {
     const int f = (int)threadIdx.x + 64 * W * j;
-    const int64_t t = min(c * kChunk + f / kRow, P.max_tokens - 1);
+    const int64_t t = min(c * kChunk + f / kRow, T_act - 1);
     vr[j] = *reinterpret_cast<const quad_t*>(vbase + t * P.v_tok + 8 * (f % kRow));
   }
   T qraw[HW][NV];
@@ -433,9 +431,7 @@ __global__ __launch_bounds__(64 * ((G + 3) / 4)) void attn_mfma_kernel(AttnParam
   for (int g = 0; g < HW; g++)
 #pragma unroll
     for (int n = 0; n < NV; n++) qraw[g][n] = reinterpret_cast<const T*>(P.q)[(int64_t)(h0 + g) * D + 64 * n + lane];
-  const int T_act = min(P.tokens_dev ? P.tokens_dev[0] + P.tokens : P.tokens, P.max_tokens);
   __builtin_amdgcn_sched_barrier(0);   // every load above is requested first
-  if (c * kChunk >= T_act) return;
   const int t = c * kChunk + lane;
   const bool valid = t < T_act;
   const int nt = min(kChunk, T_act - c * kChunk);
