@@ -1,5 +1,5 @@
-"""Decode attention outside the one-launch grids: matrix-core chunk partials and the fold
-(attn_mfma_kernel, attn_fold_kernel) bit for bit against the oracle, for every number of
+"""Decode attention outside the one-launch grids: chunk partials and the fold
+(attn_mfma_kernel, attn_kvchunk_kernel, attn_fold_kernel) bit for bit against the oracle, for every number of
 query heads per KV head, both head dimensions and KV types, capacities that end inside a
 chunk, strided caches, garbage past the count, one token and several fold blocks."""
 
@@ -57,6 +57,37 @@ def test_attention_partials_and_fold(backend, device, heads, kv_heads, dim, toke
                                    sk.ctypes.data if sinks else None, code, n, heads, kv_heads, dim, want.ctypes.data)
         got = out.cpu().view(torch.int16).numpy().view(np.uint16)
         assert_bits_equal(got, want.view(np.uint16), f"{n} tokens")
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,cap,sinks", [
+    (64, 8, 64, 4096, True),      # one launch up to 20 known chunks, then one wave per head and the fold
+    (8, 8, 64, 4160, False),      # 65 chunks: the count read before the rows
+    (256, 32, 64, 4096, True),    # more than 12288 waves: matrix-core partials, unless the host knows the count
+    (512, 64, 64, 640, False),    # 640 workgroups in one launch
+    (16, 4, 128, 8192, True),
+    (2, 1, 128, 5000, False),     # capacity inside a chunk
+    (16, 1, 64, 4200, True),      # sixteen heads, four waves
+])
+def test_counts_of_a_long_cache(backend, device, heads, kv_heads, dim, cap, sinks):
+    """Every form gives the oracle's bits on one cache and scratch, the counts going up and
+    down across the borders of the dispatch, known to the host and only on the device; each
+    call leaves the arrival counters at zero."""
+    g = rng(cap + heads)
+    q, sk = f16_normal(g, heads * dim), f16_normal(g, heads) if sinks else None
+    keys, vals = f16_normal(g, (kv_heads, cap, dim)), f16_normal(g, (kv_heads, cap, dim))
+    qd, kd, vd = (to_torch(a, device) for a in (q, keys, vals))
+    skd = to_torch(sk, device) if sinks else None
+    out = torch.empty(heads * dim, device=device, dtype=torch.float16)
+    want = np.empty(heads * dim, dtype=np.float16)
+    for n in sorted({min(cap, n) for n in (1, 64, 65, 1280, 1281, 4096, 4097, cap)}, key=lambda n: (n % 3, n)):
+        oracle.lib().tto_attention(q.ctypes.data, keys.ctypes.data, vals.ctypes.data, oracle.F16, cap * dim, dim, cap * dim,
+                                   dim, sk.ctypes.data if sinks else None, oracle.F16, n, heads, kv_heads, dim,
+                                   want.ctypes.data)
+        for count in (torch.tensor([n], dtype=torch.int32, device=device), n):
+            out.fill_(7.0)
+            backend.single_token_gqa_attention(qd, kd, vd, out, heads, kv_heads, dim, sinks=skd, active_tokens=count)
+            assert_bits_equal(from_torch_bits(out), want, f"{n} tokens, {type(count).__name__}")
+            assert not backend._attention_partials[:1024].view(torch.int32).any()
 
 
 @pytest.mark.parametrize("heads,kv_heads,dim,tokens,max_tokens", [(8, 2, 128, 130, 1000), (40, 10, 128, 64, 4500),

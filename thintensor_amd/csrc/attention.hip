@@ -17,10 +17,11 @@
 // growing cache; chunks past the count exit without work.  The count is clamped to
 // max_tokens so a runaway device counter can never read past the cache.
 //
-// Three forms, all with these bits: one launch for small grids of contiguous head_dim-64
-// caches (attn_kvchunk_kernel), matrix-core partials and a fold for everything else of
-// head_dim 64 or 128 (attn_mfma_kernel, attn_fold_kernel), scalar loads for the rest
-// (attn_partial_kernel, attn_combine_kernel).
+// Four forms, all with these bits: for contiguous head_dim-64 caches one launch of small
+// grids (attn_kvchunk_kernel), and its partials with a fold (attn_fold_kernel) of middling
+// ones; matrix-core partials (attn_mfma_kernel) and the fold for everything else of head_dim
+// 64 or 128; scalar loads for the rest (attn_partial_kernel, attn_combine_kernel).  Where the
+// host knows the count only its chunks are launched.
 #include "tt_abi_internal.h"
 #include "tt_common.h"
 
@@ -42,6 +43,7 @@ struct AttnParams {
   float* part_l;
   float* part_o;          // [heads, max_chunks, D]
   int heads, kv_heads, head_dim, max_chunks, max_tokens;
+  int grid_chunks;        // chunks launched: those of the count where the host knows it
   float scale;
   void* out;              // [heads, D]
 };
@@ -201,7 +203,13 @@ __device__ __forceinline__ float ld_dev(const float* p) {
   return __hip_atomic_load(const_cast<float*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <typename T, typename SKT, int G, bool COMBINE = true>
+//
+// Without COMBINE the partials are the result.  There a grid of many chunks may lie mostly
+// past the count, which is then read first (COUNT_FIRST, above kCountFirstChunks: 100 tokens of
+// 256 chunks, 32 / 8 heads with the o_proj GEMV: 15.5 -> 10.9 us, full 112 -> 111).
+constexpr int kCountFirstChunks = 64;
+
+template <typename T, typename SKT, int G, bool COMBINE = true, bool COUNT_FIRST = false>
 __global__ __launch_bounds__(64 * G) void attn_kvchunk_kernel(AttnParams P, int* counters) {
   constexpr int D = 64;
   const int c = blockIdx.x, kvh = blockIdx.y;
@@ -214,6 +222,7 @@ __global__ __launch_bounds__(64 * G) void attn_kvchunk_kernel(AttnParams P, int*
   __shared__ float p_s[G][kChunk];
   __shared__ int last;
   const float ninf = __builtin_bit_cast(float, 0xff800000u);
+  if (COUNT_FIRST && c * kChunk >= (P.tokens_dev ? P.tokens_dev[0] + P.tokens : P.tokens)) return;
   // every load before the active count is known (chunks below max_chunks are inside the
   // capacity): K and V pieces of the chunk, this wave's query row
   constexpr int kPer = kChunk * D / 8 / nthr;   // 16-byte pieces per thread
@@ -384,10 +393,11 @@ __global__ __launch_bounds__(64 * G) void attn_kvchunk_kernel(AttnParams P, int*
 // not.
 //
 // Partials and fold against what ran before (microseconds a call, graph-timed, caches in
-// rotation): heads / KV heads x head_dim, tokens -- 64 / 8 x 64, 16385: 42.8 -> 22.9 (one
-// wave per query head and one workgroup per KV head folding 257 chunks); 512 / 64 x 64,
-// 1025: 16.7 -> 14.8; 40 / 10 x 128, 4001: 30.8 -> 14.7; 64 / 8 x 128, 32768: 148 -> 49.5
-// (2.7 TB/s; both scalar loads before).  Past a few thousand tokens the partials bound it:
+// rotation): heads / KV heads x head_dim, tokens -- 64 / 8 x 64, 32768: 77 -> 31 (one wave
+// per query head and one workgroup per KV head folding 512 chunks); 512 / 64 x 64, 4096: 46 ->
+// 27; 40 / 10 x 128, 4001: 30.8 -> 14.7; 64 / 8 x 128, 32768: 148 -> 49.5 (2.7 TB/s; both
+// scalar loads before; they are faster only for 20 tokens or fewer, 8 / 8 x 128, 16 tokens:
+// 8.1 against 8.7).  Past a few thousand tokens the partials bound it:
 // about 16 us at 4112 waves, vector and LDS work of about 480 and 130 instructions a wave
 // and the latency of 2 x 64 dependent MFMAs rather than memory.
 typedef float acc4_t __attribute__((ext_vector_type(4)));
@@ -650,27 +660,53 @@ static bool mfma_operands(const AttnParams& P) {
          P.k_head % 8 == 0 && aligned(P.values, 16) && P.v_tok % 8 == 0 && P.v_head % 8 == 0;
 }
 
+// Chunk partials of contiguous head_dim-64 caches of whole chunks: attn_kvchunk_kernel without
+// its arrival count and combine, for the fold or for a consumer that combines the partials
+// itself (tt_attention_combine_int4_matvec; matrix-core partials were slower there below the
+// largest grids: 32 / 8 heads with the GEMV, 33 chunks 8.0 - 18.5 us against 10.0 - 20.0, 256
+// chunks, full, 112 against 111).
+template <typename T, int G>
+static int launch_kvchunk_partials(const AttnParams& P, hipStream_t st) {
+  const dim3 grid((unsigned)P.grid_chunks, (unsigned)P.kv_heads), block(64 * G);
+  if (P.grid_chunks > kCountFirstChunks)
+    hipLaunchKernelGGL((attn_kvchunk_kernel<T, f16_t, G, false, true>), grid, block, 0, st, P, nullptr);
+  else
+    hipLaunchKernelGGL((attn_kvchunk_kernel<T, f16_t, G, false, false>), grid, block, 0, st, P, nullptr);
+  return check_launch("gqa_attention_partials");
+}
+
 template <typename T, int G>
 static int launch_mfma_partials(const AttnParams& P, hipStream_t st) {
-  const dim3 grid((unsigned)P.max_chunks, (unsigned)P.kv_heads), block(64 * ((G + 3) / 4));
+  const dim3 grid((unsigned)P.grid_chunks, (unsigned)P.kv_heads), block(64 * ((G + 3) / 4));
   if (P.head_dim == 64) hipLaunchKernelGGL((attn_mfma_kernel<T, G, 64>), grid, block, 0, st, P);
   else hipLaunchKernelGGL((attn_mfma_kernel<T, G, 128>), grid, block, 0, st, P);
   return check_launch("gqa_attention");
 }
 
-// Grids that one launch serves better than partials and fold: at most one workgroup per CU
-// and 32 chunks, where the second launch costs more than the last workgroup's fold (one
-// launch against two: 32 / 8 heads, 513 tokens 6.3 against 8.4 us, 64 / 8, 1025 tokens 7.8
-// against 8.4; 64 KV heads of 17 chunks 16.7 against 14.8, 8 of 65 chunks 15.5 against 9.1).
+// Grids that one launch serves better than partials and fold, where the second launch costs
+// more than the last workgroup's fold: one workgroup per CU and, of a count the host knows, 20
+// chunks (64 / 8 heads: 16 chunks 7.7 us in one launch against 7.8 in two, 32 chunks 10.0
+// against 8.7); a count that only the device knows is taken to be half the capacity or more
+// (33 chunks: 64 tokens 6.2 against 7.3 us, 1000 tokens 8.0 against 7.8, all 11.9 against
+// 8.9).  Several workgroups per CU while their fold is short (512 / 64 heads: 9 chunks, 288
+// tokens, 8.5 against 9.8 us, full 11.4 against 11.0; 16 chunks 17.9 against 12.5).
 static bool one_launch_grid(const AttnParams& P) {
-  return P.max_chunks <= 32 && (int64_t)P.max_chunks * P.kv_heads <= 256;
+  const int64_t groups = (int64_t)P.grid_chunks * P.kv_heads;
+  return P.grid_chunks <= 10 ? groups <= 640 : P.grid_chunks <= (P.tokens_dev ? 32 : 20) && groups <= 256;
 }
+
+// Partials of one wave per query head: where the chip holds most of the waves at once they
+// end sooner than the matrix-core partials, whose two chains of 64 dependent MFMAs take about
+// 1.5 us more than fused multiply-adds (with the fold, 64 / 8 heads: 33 chunks 10.4 -> 8.9
+// us, 192 chunks 18.3 -> 17.3, 256 chunks 19.5 -> 20.4; 512 / 64 heads: 24 chunks 17.1 ->
+// 15.6, 32 chunks 17.1 -> 17.8; 100 tokens of 64 chunks, 64 / 8 heads, 10.5 -> 8.6).
+static bool head_wave_grid(const AttnParams& P) { return (int64_t)P.grid_chunks * P.heads <= 12288; }
 
 template <typename T, int G>
 static int launch_attn(const AttnParams& P, int sink_dtype, bool contiguous64, int* counters, hipStream_t st) {
   if constexpr (G <= 8) {
     if (contiguous64 && counters != nullptr && one_launch_grid(P)) {
-      const dim3 block(64 * G), grid((unsigned)P.max_chunks, (unsigned)P.kv_heads);
+      const dim3 block(64 * G), grid((unsigned)P.grid_chunks, (unsigned)P.kv_heads);
       switch (sink_dtype) {
         case TT_BF16: hipLaunchKernelGGL((attn_kvchunk_kernel<T, bf16_t, G>), grid, block, 0, st, P, counters); break;
         case TT_F32: hipLaunchKernelGGL((attn_kvchunk_kernel<T, float, G>), grid, block, 0, st, P, counters); break;
@@ -678,12 +714,16 @@ static int launch_attn(const AttnParams& P, int sink_dtype, bool contiguous64, i
       }
       return check_launch("gqa_attention");
     }
+    if (contiguous64 && head_wave_grid(P)) {
+      const int rc = launch_kvchunk_partials<T, G>(P, st);
+      return rc ? rc : launch_fold<T>(P, sink_dtype, st);
+    }
   }
   if (mfma_operands(P)) {
     const int rc = launch_mfma_partials<T, G>(P, st);
     return rc ? rc : launch_fold<T>(P, sink_dtype, st);
   }
-  hipLaunchKernelGGL((attn_partial_kernel<T, G>), dim3(P.max_chunks, P.kv_heads), dim3(64), 0, st, P);
+  hipLaunchKernelGGL((attn_partial_kernel<T, G>), dim3(P.grid_chunks, P.kv_heads), dim3(64), 0, st, P);
   int rc = check_launch("gqa_attention");
   if (rc) return rc;
   switch (sink_dtype) {
@@ -702,17 +742,6 @@ using namespace tt;
 extern "C" int tt_attention_scratch_floats(int64_t heads, int64_t max_tokens, int64_t head_dim) {
   const int64_t chunks = (max_tokens + kChunk - 1) / kChunk;
   return (int)(kAttnCounters + heads * chunks * (2 + head_dim));
-}
-
-// Chunk partials only (contiguous head_dim-64 caches, whole-chunk capacity, no sinks):
-// the one-launch kernel without its arrival count and combine, for a consumer that
-// combines the partials itself (tt_attention_combine_int4_matvec).
-template <typename T, int G>
-static int launch_attn_partials(const AttnParams& P, hipStream_t st) {
-  if (!one_launch_grid(P)) return launch_mfma_partials<T, G>(P, st);
-  hipLaunchKernelGGL((attn_kvchunk_kernel<T, f16_t, G, false>), dim3((unsigned)P.max_chunks, (unsigned)P.kv_heads),
-                     dim3(64 * G), 0, st, P, nullptr);
-  return check_launch("gqa_attention_partials");
 }
 
 extern "C" int tt_single_token_gqa_attention_partials(const void* q, const void* keys, const void* values, int dtype,
@@ -744,16 +773,17 @@ extern "C" int tt_single_token_gqa_attention_partials(const void* q, const void*
   P.part_o = scratch + 2 * heads * chunks;
   P.heads = (int)heads; P.kv_heads = (int)kv_heads; P.head_dim = (int)head_dim; P.max_chunks = (int)chunks;
   P.max_tokens = (int)max_tokens;
+  P.grid_chunks = (int)(tokens_dev ? chunks : (tokens + kChunk - 1) / kChunk);
   P.scale = (float)(1.0 / __builtin_sqrt((double)head_dim));
   P.out = nullptr;
   hipStream_t st = static_cast<hipStream_t>(stream);
   auto by_g = [&](auto t) -> int {
     using T = decltype(t);
     switch (G) {
-      case 1: return launch_attn_partials<T, 1>(P, st);
-      case 2: return launch_attn_partials<T, 2>(P, st);
-      case 4: return launch_attn_partials<T, 4>(P, st);
-      default: return launch_attn_partials<T, 8>(P, st);
+      case 1: return launch_kvchunk_partials<T, 1>(P, st);
+      case 2: return launch_kvchunk_partials<T, 2>(P, st);
+      case 4: return launch_kvchunk_partials<T, 4>(P, st);
+      default: return launch_kvchunk_partials<T, 8>(P, st);
     }
   };
   if (dtype == TT_F16) return by_g(f16_t{});
@@ -789,6 +819,7 @@ extern "C" int tt_single_token_gqa_attention(const void* q, const void* keys, co
   P.part_o = scratch + 2 * heads * chunks;
   P.heads = (int)heads; P.kv_heads = (int)kv_heads; P.head_dim = (int)head_dim; P.max_chunks = (int)chunks;
   P.max_tokens = (int)max_tokens;
+  P.grid_chunks = (int)(tokens_dev ? chunks : (tokens + kChunk - 1) / kChunk);
   P.scale = (float)(1.0 / __builtin_sqrt((double)head_dim));
   P.out = out;
   const int G = (int)(heads / kv_heads);
