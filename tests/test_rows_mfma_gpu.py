@@ -1,6 +1,6 @@
-"""Several activation rows on the binary32 matrix cores (rows_mfma.hip): fp16 GEMV + bias,
-the fp16 lm_head argmax and the fp8 GEMM must give every row the single-row operator's
-bits, at the edges of the row tiles (16 or 32 weight rows, passes of 32 activation rows,
+"""Several activation rows on the binary32 matrix cores (rows_mfma.hip) and, where those are
+slower (few weight rows), as slots of the single-row kernel: fp16 GEMV + bias, the fp16
+lm_head argmax and the fp8 GEMM must give every row the single-row operator's bits, at the edges of the row tiles (16 or 32 weight rows, passes of 32 activation rows,
 the 4-, 8- and 16-row forms), of the chunk groups (ragged last group, each lanes-per-row
 value) and of the tile schedule (more tiles than workgroups, one tile, two row tiles per
 wave)."""
@@ -81,3 +81,59 @@ def test_fp8_rows(backend, device, m, rows, cols):
     for r in range(m):
         want = oracle.gemv("fp8", "row", bits, scales, x[r], cols=cols, lpr=lanes(cols), s_row=1)
         assert_bits_equal(from_torch_bits(out[r]), want, f"row {r}")
+
+
+# Sizes that the matrix-core kernel serves rather than slots of the single-row kernel, compared
+# with the single-row operators (which other tests compare with the oracle): 16, 32 and 64
+# lanes per row in four- and eight-wave workgroups, each activation form.
+@pytest.mark.parametrize("m,rows,cols", [
+    (3, 1840, 2880), (4, 1375, 8192),     # four rows of activations, eight waves
+    (5, 4200, 2048), (8, 4130, 2880),     # eight rows, four waves, 64 and 32 lanes
+    (8, 1124, 4096), (8, 1125, 4096),     # the last size of the slots, the first past it
+    (12, 1050, 96), (16, 4113, 4096),     # sixteen rows, 16 and 64 lanes
+    (17, 5000, 2880), (32, 5000, 2048),   # two activation tiles, more tiles than CUs
+    (33, 930, 5152), (35, 1000, 16384),   # a second pass of one and of three rows
+    (3, 32801, 512), (20, 1000, 32768),
+    (64, 64, 5120), (31, 780, 32768),     # slots
+    (2, 3300, 5152), (2, 2056, 8192), (2, 2048, 8192),   # two rows: engine, engine, slots
+])
+def test_bias_rows_match_single_rows(backend, device, m, rows, cols):
+    g = torch.Generator(device=device).manual_seed(rows + cols + m)
+    w, x, bias = (torch.randn(s, generator=g, device=device).mul_(f).half()
+                  for s, f in (((rows, cols), 0.05), ((m, cols), 1.0), ((rows,), 1.0)))
+    out, one = (torch.empty((m, rows), device=device, dtype=torch.float16) for _ in range(2))
+    backend.matvec_bias_rows(w, bias, x, out)
+    for t in range(m):
+        backend.multi_matvec_bias((w,), (bias,), x[t], one[t])
+    assert torch.equal(out.view(torch.int16), one.view(torch.int16))
+
+
+@pytest.mark.parametrize("m,rows,cols", [(3, 32801, 2048), (4, 32801, 2880), (7, 32801, 2880), (16, 32801, 2048),
+                                         (16, 32801, 2880), (20, 32801, 2048), (32, 5000, 2880), (32, 5000, 2048),
+                                         (64, 5000, 4096)])
+def test_lm_head_matches_single_rows(backend, device, m, rows, cols):
+    """Two weight tiles per wave at each lanes-per-row value, and two activation tiles in four-wave
+    workgroups."""
+    g = torch.Generator(device=device).manual_seed(rows + cols + m)
+    w = torch.randn((rows, cols), generator=g, device=device).mul_(0.05).half()
+    x = torch.randn((m, cols), generator=g, device=device).half()
+    logits, one = (torch.empty((m, rows), device=device, dtype=torch.float16) for _ in range(2))
+    idx = backend.matvec_argmax_batched(w, x, logits)
+    for t in range(m):
+        assert int(backend.matvec_argmax_tensor(w, x[t])) == int(idx[t]), f"row {t}"
+        one[t] = backend.logits_buffer(rows, torch.float16)
+    assert torch.equal(logits.view(torch.int16), one.view(torch.int16))
+
+
+@pytest.mark.parametrize("m,rows,cols", [(4, 4200, 4096), (12, 4200, 4096), (4, 32900, 4096), (12, 32900, 4096),
+                                         (7, 32900, 2816), (8, 1124, 2048), (8, 1125, 2048), (15, 900, 8192)])
+def test_fp8_rows_match_single_rows(backend, device, m, rows, cols):
+    g = torch.Generator(device=device).manual_seed(rows + cols + m)
+    w = torch.randn((rows, cols), generator=g, device=device).mul_(100).clamp_(-448, 448).to(torch.float8_e4m3fn)
+    scales = torch.rand(rows, generator=g, device=device) * 0.01 + 1e-3
+    x = torch.randn((m, cols), generator=g, device=device).half()
+    out, one = (torch.empty((m, rows), device=device, dtype=torch.float16) for _ in range(2))
+    backend.scaled_batched_matvec(w, scales, x, out)
+    for t in range(m):
+        backend.scaled_matvec(w, scales, x[t], one[t])
+    assert torch.equal(out.view(torch.int16), one.view(torch.int16))

@@ -772,6 +772,8 @@ extern "C" int tt_scaled_batched_matvec(const void* weight, int64_t w_row_bytes,
                  static_cast<uint16_t*>(out), out_row, (int)m, (int)rows, (int)cols};
     return launch_mfma<WFmt::kFp8Row>(P, st, what);
   }
+  if (m >= kRowsMfmaMin && rows * w_row_bytes < (1LL << 31) && row_slots_better(m, rows, cols))
+    return scaled_slots_fp8(weight, w_row_bytes, scales, x, x_row, out, out_row, m, rows, cols, st, what);
   if (m >= kRowsMfmaMin && rows_mfma_fits(w_row_bytes, x_row))
     return rows_mfma_fp8({weight, w_row_bytes, scales, nullptr, x, x_row, out, out_row, m, rows, cols}, st, what);
   if (m == 1)   // one row: the single-row GEMV itself (its lean kernel; the same bits as a row of the engine)

@@ -50,6 +50,24 @@ static int scaled_matvec_fmt(const void* weight, int64_t w_row_bytes, const void
   return launch_types<F, SMode::kRow, float, 4>(x_dtype, out_dtype, Lg, lpr, P, 1, st, what);
 }
 
+namespace tt {
+int scaled_slots_fp8(const void* weight, int64_t w_row_bytes, const float* scales, const void* x, int64_t x_row, void* out,
+                     int64_t out_row, int64_t m, int64_t rows, int64_t cols, hipStream_t st, const char* what) {
+  LeanParams L{};
+  L.w = static_cast<const uint8_t*>(weight);
+  L.s = scales;
+  L.x = x;
+  L.out = out;
+  L.x_slot = x_row;
+  L.out_slot = out_row;
+  L.w_row = (uint32_t)w_row_bytes;
+  L.s_row = 1;
+  L.rows = (int)rows;
+  L.cols = (int)cols;
+  return lean_launch<Fmt::kFp8, SMode::kRow, float, 1>(TT_F16, tt_gemv_lanes_per_row(cols / 32, 1), L, (int)m, st, what);
+}
+}  // namespace tt
+
 static int scaled_matvec_impl(const void* weight, int w_format, int64_t w_row_bytes, const void* scales,
                               int scale_dtype, int64_t s_stride, const void* x, int x_dtype, void* out, int out_dtype,
                               int64_t rows, int64_t cols, void* stream) {
@@ -139,11 +157,15 @@ extern "C" int tt_matvec_bias_rows(const void* weight, int w_dtype, int64_t w_ro
     return TT_OK;
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // the GEMV engine takes up to 4096 columns (its activation rows share LDS), the matrix-core
-  // kernel any width
-  if (w_dtype == TT_F16 && x_dtype == TT_F16 &&
-      (cols <= 4096 || (m >= kRowsMfmaMin && rows_mfma_fits(w_row * 2, x_row))))
-    return dense_bias_rows_f16(weight, w_row, bias, x, x_row, out, out_row, m, rows, cols, st);
+  if (w_dtype == TT_F16 && x_dtype == TT_F16) {
+    // from three rows the matrix-core kernel or slots; two rows on the GEMV engine, past 4096
+    // columns only with a weight that outgrows the caches (slots read it twice: 2880 x 8192 14.8
+    // us as slots, 14.6 on the engine, 8192 x 5120 27.7 and 19.7; 2048 x 8192 10.6 and 11.3)
+    const bool matrix = m >= kRowsMfmaMin && rows_mfma_fits(w_row * 2, x_row);
+    const bool engine = cols <= 4096 || (m == 2 && cols <= 8192 && rows * cols > (1 << 24));
+    if (matrix ? !row_slots_better(m, rows, cols) : engine)
+      return dense_bias_rows_f16(weight, w_row, bias, x, x_row, out, out_row, m, rows, cols, st);
+  }
   // rows of the batch are slots of the lean kernel (blockIdx.y), each with its own
   // activation and output row; the arithmetic per row is the single-row kernel's
   LeanParams L{};

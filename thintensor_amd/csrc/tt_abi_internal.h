@@ -46,6 +46,11 @@ inline bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintp
 int dense_bias_rows_f16(const void* weight, int64_t w_row, const void* bias, const void* x, int64_t x_row, void* out,
                         int64_t out_row, int64_t m, int64_t rows, int64_t cols, hipStream_t st);
 
+// y[r] = (W x[r]) scale for m fp16 activation rows as slots of the single-row fp8 kernel
+// (gemv_dense.hip).  Operands checked by the caller, 32-bit offsets (rows w_row_bytes < 2^31).
+int scaled_slots_fp8(const void* weight, int64_t w_row_bytes, const float* scales, const void* x, int64_t x_row, void* out,
+                     int64_t out_row, int64_t m, int64_t rows, int64_t cols, hipStream_t st, const char* what);
+
 // y[r] = W x[r] for m fp16 activation rows on the binary32 matrix cores, row r with the
 // bits of the single-row GEMV (rows_mfma.hip): fp16 weights with an optional fp16 bias, fp8
 // weights with fp32 row scales, and the fp16 lm_head with its argmax.  Passes of kRowsPass
@@ -56,6 +61,20 @@ constexpr int kRowsPass = 32;
 // fp8 17920 x 5120 39 against 24); at two, one launch each, the engine is as fast or faster
 // (268 against 263 us, 18.8 against 21.2).
 constexpr int kRowsMfmaMin = 3;
+// Whether the activation rows run sooner as slots of the single-row lean kernel (a grid row
+// each, the same bits): their time grows with rows x m, that of a matrix-core pass of up to 4,
+// 8, 16 or 32 rows hardly does while there are fewer row tiles than CUs.  Break-even of fp16
+// matrices of 2048 to 32768 columns; us as slots against matrix cores: 64 x 5120, 64 rows 5.2
+// against 36.9; 1024 x 5120, 3 rows 6.3 against 8.5, 8 rows 9.2 against 11.4, 16 rows 14.1
+// against 13.3; 1536 x 5120, 4 rows 9.6 against 8.9; 768 x 8192, 32 rows 27 against 29; 2880 x
+// 5120, 8 rows 31 against 12; a fifth earlier where the slots' weight reads miss the L2s
+// (1280 x 32768, 4 rows 46 against 34).  (fp8 breaks even later: 2048 x 5120, 8 rows 1.2 times
+// as fast as slots, 2880 x 5120 0.85 times.)
+inline bool row_slots_better(int64_t m, int64_t rows, int64_t cols) {
+  const int64_t tail = m % kRowsPass;
+  const int64_t even = m / kRowsPass * 25000 + (tail == 0 ? 0 : tail <= 4 ? 5500 : tail <= 8 ? 9000 : tail <= 16 ? 12500 : 25000);
+  return rows * m < (cols > 16384 ? even / 5 * 4 : even);
+}
 struct RowsArgs {
   const void* weight;
   int64_t w_row_bytes;
