@@ -10,7 +10,7 @@ import pytest
 import torch
 
 import oracle
-from tests.helpers import f16_normal, from_torch_bits, rng, to_torch
+from tests.helpers import bf16_bits, bf16_to_f32, f16_normal, from_torch_bits, rng, to_torch
 from tests.test_gemv_gpu import assert_bits_equal
 from thintensor_amd import _lib
 
@@ -115,3 +115,45 @@ def test_rows_past_the_count_need_not_exist(backend, device, heads, kv_heads, di
             torch.cuda.current_stream(device).cuda_stream)
         _lib.check(rc, "single_token_gqa_attention")
         assert_bits_equal(from_torch_bits(out), want, "device count" if dev else "host count")
+
+
+@pytest.mark.parametrize("kind", ["tiny values", "late weights", "inf and nan"])
+@pytest.mark.parametrize("dim,cap", [(128, 200), (64, 200), (64, 192), (64, 4096), (96, 192)])
+def test_subnormals_and_non_finite_values(backend, device, kind, dim, cap):
+    """Every form keeps binary32 subnormals (the oracle's fmaf chains do): values whose products
+    with the weights and their sums are subnormal, and weights near the smallest normal number
+    on the only tokens with values; infinities and NaN of K and V rows inside the count reach
+    the same outputs."""
+    heads, kv_heads, tokens = 16, 4, 150
+    g = rng(dim + cap + len(kind))
+    q = g.standard_normal((heads, dim))
+    keys, vals = g.standard_normal((kv_heads, cap, dim)), g.standard_normal((kv_heads, cap, dim))
+    if kind == "tiny values":
+        vals *= 2.0 ** -g.integers(122, 133, (kv_heads, cap, 1))
+    elif kind == "late weights":
+        # scores from 0 down to -87 below the first token's; values from token 100 on
+        q[:] = 1.0
+        keys[:] = -np.linspace(0.0, 86.5, tokens).repeat(cap // tokens + 1)[:cap, None] / np.sqrt(dim)
+        keys[:, 140:tokens] = -86.0 / np.sqrt(dim)
+        vals[:, :100] = 0.0
+        vals[:, 100:] *= 2.0 ** -g.integers(0, 8, (kv_heads, cap - 100, 1))
+        vals[:, 100:140] = 0.0
+    else:
+        keys[1, 70, 3], keys[2, 5, 0], vals[3, 149, 7], vals[3, 0, 9] = np.nan, np.inf, -np.inf, np.nan
+    q, keys, vals = (bf16_bits(a.astype(np.float32)) for a in (q, keys, vals))
+    out = torch.empty(heads * dim, device=device, dtype=torch.bfloat16)
+    want = np.empty(heads * dim, dtype=np.uint16)
+    oracle.lib().tto_attention(q.ctypes.data, keys.ctypes.data, vals.ctypes.data, oracle.BF16, cap * dim, dim, cap * dim, dim,
+                               None, oracle.BF16, tokens, heads, kv_heads, dim, want.ctypes.data)
+    w = bf16_to_f32(want)
+    if kind == "inf and nan":
+        assert np.isnan(w).any() and np.isinf(w).any() and np.isfinite(w).any()
+    else:
+        assert ((w != 0) & (np.abs(w) < 2.0 ** -126)).any()
+    qd, kd, vd = (to_torch(a, device, True) for a in (q, keys, vals))
+    count = torch.tensor([tokens], dtype=torch.int32, device=device)
+    backend.single_token_gqa_attention(qd.view(-1), kd, vd, out, heads, kv_heads, dim, active_tokens=count)
+    got = from_torch_bits(out)
+    nan = np.isnan(w)
+    assert np.array_equal(np.isnan(bf16_to_f32(got)), nan)
+    assert_bits_equal(np.where(nan, 0, got).astype(np.uint16), np.where(nan, 0, want).astype(np.uint16), kind)
