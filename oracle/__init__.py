@@ -53,6 +53,8 @@ def _register_extra(L: ctypes.CDLL) -> None:
         fn.restype = _I
     L.tto_argmax.argtypes = [_P, _I, _L]
     L.tto_argmax.restype = _L
+    L.tto_residual_round_mismatches.argtypes = [ctypes.c_int32, ctypes.c_int32]
+    L.tto_residual_round_mismatches.restype = _L
 
 
 _F = ctypes.c_float

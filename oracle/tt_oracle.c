@@ -657,3 +657,40 @@ int64_t tto_argmax(const void* logits, int dt, int64_t n) {
   }
   return bi;
 }
+
+/* ------------------------------------------------------------ symmetric INT4 rounding */
+
+static float float_step(float f, int k) {
+  int32_t u;
+  memcpy(&u, &f, 4);
+  u += k;
+  memcpy(&f, &u, 4);
+  return f;
+}
+
+/* How often rint of x / s by reciprocal and one residual step (round_codes of quantize.hip)
+ * differs from rintf(x / s), over the 24-bit significands [lo, hi) of s: the reciprocal r0 up
+ * to two floats from 1 / s, refined by one Newton step, x up to four floats from every tie
+ * up to 8.5 (the only places where an error of an ulp of the quotient shows). */
+int64_t tto_residual_round_mismatches(int32_t lo, int32_t hi) {
+  int64_t bad = 0;
+#pragma omp parallel for schedule(static) reduction(+ : bad)
+  for (int32_t sig = lo; sig < hi; sig++) {
+    const float s = (float)sig, exact = 1.0f / s;
+    float last = 0.0f;
+    for (int k = -2; k <= 2; k++) {
+      const float r0 = float_step(exact, k);
+      const float r = fmaf(fmaf(-s, r0, 1.0f), r0, r0);
+      if (r == last) continue;
+      last = r;
+      for (int h = 1; h <= 17; h += 2) {
+        const float tie = (float)((double)sig * h * 0.5);
+        for (int d = -4; d <= 4; d++) {
+          const float x = float_step(tie, d), t = x * r;
+          bad += rintf(fmaf(fmaf(-t, s, x), r, t)) != rintf(x / s);
+        }
+      }
+    }
+  }
+  return bad;
+}

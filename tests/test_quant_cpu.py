@@ -214,3 +214,13 @@ def test_planted_mistakes_are_caught(V, monkeypatch):
     assert not np.array_equal(Q.floor_log2(amax), Q.floor_log2((amax / np.float32(1.5)).astype(np.float32)))
     p1, s1 = Q.dense_to_lowbit(x, 1)
     assert not same(s1, V["dense_q2.out_scales"])
+
+
+def test_residual_step_rounds_as_the_division():
+    """The symmetric INT4 kernel takes rint(x / s) from a refined reciprocal and one residual step
+    for every significand of the scale but all ones, which it divides: tried for all of them
+    next to every tie."""
+    from oracle import lib
+
+    assert lib().tto_residual_round_mismatches(0x800000, 0xFFFFFF) == 0
+    assert lib().tto_residual_round_mismatches(0xFFFFFF, 0x1000000) > 0

@@ -13,14 +13,17 @@
 //   tt_quantize_dense_lowbit     quantize_dense_to_mxfp_lowbit_cpu :398-491
 //   tt_pack_mxfp4_ternary        quantize_mxfp4_to_ternary_cpu :494-583
 //
-// Arithmetic (restated in oracle/quant.py): every elementwise step is the reference's
-// binary32 operation in its order (IEEE division, round-half-even rounding); every sum
-// over a quantization group is taken in binary64 -- each lane adds its elements in
-// index order from +0, then the lane partials are folded in halves (lane bit 32
+// Arithmetic (restated in oracle/quant.py): every elementwise step has the result of the
+// reference's binary32 operation in its order (IEEE division, round-half-even rounding);
+// every sum over a quantization group is taken in binary64 -- each lane adds its elements
+// in index order from +0, then the lane partials are folded in halves (lane bit 32
 // first for a 64-lane group, bit 16 first for a 32-lane MX group) -- and rounded once
 // to binary32; ceil/floor of log2 come from the binary exponent.  One wave owns one
 // quantization group (int4) or two 32-element MX groups (one per half-wave), so no
-// group needs more than cross-lane moves.
+// group needs more than cross-lane moves.  Symmetric INT4 of most layouts
+// (int4_sym_kernel) puts several groups in a wave, sums in any order and partly in
+// binary32 where that is exact, and takes quotients' roundings from a reciprocal, all
+// with the same results; the reasons stand there.
 #include <type_traits>
 
 #include "tt_abi_internal.h"
@@ -151,10 +154,12 @@ struct Q4Params {
 // order.)
 //
 // rint(x / s) is rint of a product with the reciprocal and one residual step, five operations
-// of one rounding each.  Its value next to every half-integer up to 8.5 equals that of the
-// quotient for every 24-bit significand of s but all ones and every reciprocal within an ulp of
-// 1 / s (all of them tried, x up to four ulps from the tie); elsewhere the step is within an ulp
-// of the quotient and past 8.5 both clamp alike.  Groups where a step could overflow or the
+// of one rounding each.  The reciprocal is the hardware's, within an ulp of 1 / s, after one
+// Newton step.  Next to every half-integer up to 8.5 the value then equals that of the
+// quotient for every 24-bit significand of s but all ones: all of them tried, with starting
+// reciprocals up to two floats from 1 / s and x up to four floats from the tie
+// (tto_residual_round_mismatches, a CPU test).  Elsewhere the step is within an ulp of the
+// quotient and past 8.5 both clamp alike.  Groups where a step could overflow or the
 // reciprocal is not normal, and that one significand, divide.
 //
 // Bound by the vector units for 16-bit sources, by HBM for binary32.  17920 x 5120, group 128,
