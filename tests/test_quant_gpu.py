@@ -357,11 +357,12 @@ def test_int4_symmetric_scale_significands(affine_env, mode):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-def test_int4_symmetric_pieces_per_thread(affine_env, dtype):
+@pytest.mark.parametrize("rows", [8197, 10241])      # 33 groups of eight pieces a row: below and above 2621440
+def test_int4_symmetric_pieces_per_thread(affine_env, rows, dtype):
     """Large 16-bit matrices take several pieces per thread: the same codes and scales as
     their row blocks, which take one (compared with the oracle above)."""
     affine_env(False)
-    w = (torch.randn((8197, 2056), generator=torch.Generator().manual_seed(5)) * 0.02).to(dtype).cuda()
+    w = (torch.randn((rows, 2056), generator=torch.Generator().manual_seed(5)) * 0.02).to(dtype).cuda()
     got = TQ.quantize_to_int4_cpu(w, group_size=64)
     parts = [TQ.quantize_to_int4_cpu(w[r:r + 1000], group_size=64) for r in range(0, len(w), 1000)]
     assert torch.equal(got[0], torch.cat([p[0] for p in parts]))

@@ -827,12 +827,13 @@ extern "C" int tt_quantize_int4(const void* src, int src_dtype, int64_t rows, in
           else hipLaunchKernelGGL((int4_sym_kernel<ST, GL, false, NP>), grid, dim3(256), 0, st, P, (int)ppr);
           return check_launch(what);
         };
-        // four pieces per thread pay for 16-bit sources of large matrices: 17920 x 5120 bf16 68 us
-        // with one, 62 with two or eight, 60 with four; 5000 x 4096 18.1, 17.7 (two), 18.4 (four);
-        // 2048 x 2048 5.6 against 6.9.  binary32 sources, two loads a piece: 77 - 80 us against
-        // 81 - 84, 20.4 against 21.9, 6.7 against 8.4
+        // four pieces per thread pay for 16-bit sources of large matrices (bf16, group 128, one
+        // piece against four: 2048 x 8200 14.7 us, 15.6; 5000 x 4096 17.0, 17.1; 6000 x 4096 19.5,
+        // 19.3; 8192 x 4096 26.1, 24.4; 17920 x 5120 63.5, 57.6, two or eight 62).  binary32
+        // sources, two loads a piece, take one: 17920 x 5120 77 - 80 us against 81 - 84, 5000 x
+        // 4096 20.4 against 21.9, 2048 x 2048 6.7 against 8.4
         if constexpr (sizeof(ST) == 2) {
-          if (pieces >= 256 * 8192) return launch(std::integral_constant<int, kQ4Pieces>{});
+          if (pieces >= 256 * 10240) return launch(std::integral_constant<int, kQ4Pieces>{});
         }
         return launch(std::integral_constant<int, 1>{});
       };
