@@ -203,10 +203,11 @@ __device__ __forceinline__ float ld_dev(const float* p) {
   return __hip_atomic_load(const_cast<float*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-//
-// Without COMBINE the partials are the result.  There a grid of many chunks may lie mostly
-// past the count, which is then read first (COUNT_FIRST, above kCountFirstChunks: 100 tokens of
-// 256 chunks, 32 / 8 heads with the o_proj GEMV: 15.5 -> 10.9 us, full 112 -> 111).
+// Grids of at most kOneLaunchChunks chunks combine.  Without COMBINE the partials are the
+// result; there a grid of many chunks may lie mostly past the count, which is then read first
+// (COUNT_FIRST, above kCountFirstChunks: 100 tokens of 256 chunks, 32 / 8 heads with the o_proj
+// GEMV: 15.5 -> 10.9 us, full 112 -> 111).
+constexpr int kOneLaunchChunks = 32;
 constexpr int kCountFirstChunks = 64;
 
 template <typename T, typename SKT, int G, bool COMBINE = true, bool COUNT_FIRST = false>
@@ -316,58 +317,37 @@ __global__ __launch_bounds__(64 * G) void attn_kvchunk_kernel(AttnParams P, int*
   __syncthreads();
   if (!last) return;
 
-  // ---- combine of query head h in chunk order (combine_head's arithmetic); the
-  // first 64 chunks' (m, l) and the first kBlk chunks' partial rows are requested together
-  // with the sink, one round trip, before the maximum is formed
-  constexpr int kBlk = 32;
+  // ---- combine of query head h in chunk order (combine_head's arithmetic); (m, l) and the
+  // partial rows of every chunk are requested together with the sink, one round trip, before
+  // the maximum is formed
   const float* pm = P.part_m + (int64_t)h * P.max_chunks;
   const float* pl = P.part_l + (int64_t)h * P.max_chunks;
   const float* po = P.part_o + (int64_t)h * P.max_chunks * D + lane;
   const bool has_sink = P.sinks != nullptr;
-  const float m0 = lane < nc ? ld_dev(pm + lane) : ninf;
-  const float l0 = lane < nc ? ld_dev(pl + lane) : 0.0f;
-  float ov0[kBlk];
+  const float mc = lane < nc ? ld_dev(pm + lane) : ninf;
+  const float lv = lane < nc ? ld_dev(pl + lane) : 0.0f;
+  float ov[kOneLaunchChunks];
 #pragma unroll
-  for (int u = 0; u < kBlk; u++) ov0[u] = u < nc ? ld_dev(po + (int64_t)u * D) : 0.0f;
+  for (int u = 0; u < kOneLaunchChunks; u++) ov[u] = u < nc ? ld_dev(po + (int64_t)u * D) : 0.0f;
   const float sink = has_sink ? to_f32(reinterpret_cast<const SKT*>(P.sinks)[h]) : 0.0f;
-  float M = has_sink ? sink : ninf;
-  for (int c0 = 0; c0 < nc; c0 += 64) {
-    float mm = c0 == 0 ? m0 : (c0 + lane < nc ? ld_dev(pm + c0 + lane) : ninf);
-    mm = fmaxf(mm, xor_partner<1>(mm));
-    mm = fmaxf(mm, xor_partner<2>(mm));
-    mm = fmaxf(mm, xor_partner<4>(mm));
-    mm = fmaxf(mm, xor_partner<8>(mm));
-    mm = fmaxf(mm, xor_partner<16>(mm));
-    mm = fmaxf(mm, xor_partner<32>(mm));
-    M = fmaxf(M, mm);
-  }
+  float M = mc;
+  M = fmaxf(M, xor_partner<1>(M));
+  M = fmaxf(M, xor_partner<2>(M));
+  M = fmaxf(M, xor_partner<4>(M));
+  M = fmaxf(M, xor_partner<8>(M));
+  M = fmaxf(M, xor_partner<16>(M));
+  M = fmaxf(M, xor_partner<32>(M));
+  if (has_sink) M = fmaxf(sink, M);
   float den = has_sink ? exp_f32(sink - M) : 0.0f;
   float acc = 0.0f;
-  for (int c0 = 0; c0 < nc; c0 += 64) {
-    const int n = min(64, nc - c0);
-    const float e = c0 + lane < nc ? exp_f32((c0 == 0 ? m0 : ld_dev(pm + c0 + lane)) - M) : 0.0f;
-    const float lv = c0 + lane < nc ? (c0 == 0 ? l0 : ld_dev(pl + c0 + lane)) : 0.0f;
-    for (int c1 = 0; c1 < n; c1 += kBlk) {
-      float ov[kBlk];
-      if (c0 == 0 && c1 == 0) {
+  const float e = lane < nc ? exp_f32(mc - M) : 0.0f;
 #pragma unroll
-        for (int u = 0; u < kBlk; u++) ov[u] = ov0[u];
-      } else {
-#pragma unroll
-        for (int u = 0; u < kBlk; u++) {
-          const int cc = c0 + c1 + u;
-          ov[u] = cc < nc ? ld_dev(po + (int64_t)cc * D) : 0.0f;
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < kBlk; u++) {
-        if (c1 + u < n) {
-          const float ec = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, e), c1 + u));
-          const float lc = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lv), c1 + u));
-          den = __builtin_fmaf(lc, ec, den);
-          acc = __builtin_fmaf(ov[u], ec, acc);
-        }
-      }
+  for (int u = 0; u < kOneLaunchChunks; u++) {
+    if (u < nc) {
+      const float ec = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, e), u));
+      const float lc = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lv), u));
+      den = __builtin_fmaf(lc, ec, den);
+      acc = __builtin_fmaf(ov[u], ec, acc);
     }
   }
   store<T>(reinterpret_cast<T*>(P.out) + (int64_t)h * D + lane, acc / den);
@@ -692,7 +672,7 @@ static int launch_mfma_partials(const AttnParams& P, hipStream_t st) {
 // tokens, 8.5 against 9.8 us, full 11.4 against 11.0; 16 chunks 17.9 against 12.5).
 static bool one_launch_grid(const AttnParams& P) {
   const int64_t groups = (int64_t)P.grid_chunks * P.kv_heads;
-  return P.grid_chunks <= 10 ? groups <= 640 : P.grid_chunks <= (P.tokens_dev ? 32 : 20) && groups <= 256;
+  return P.grid_chunks <= 10 ? groups <= 640 : P.grid_chunks <= (P.tokens_dev ? kOneLaunchChunks : 20) && groups <= 256;
 }
 
 // Partials of one wave per query head: where the chip holds most of the waves at once they
