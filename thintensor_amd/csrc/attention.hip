@@ -672,7 +672,8 @@ static int launch_mfma_partials(const AttnParams& P, hipStream_t st) {
 // tokens, 8.5 against 9.8 us, full 11.4 against 11.0; 16 chunks 17.9 against 12.5).
 static bool one_launch_grid(const AttnParams& P) {
   const int64_t groups = (int64_t)P.grid_chunks * P.kv_heads;
-  return P.grid_chunks <= 10 ? groups <= 640 : P.grid_chunks <= (P.tokens_dev ? kOneLaunchChunks : 20) && groups <= 256;
+  if (P.grid_chunks <= 10) return 2 * groups <= 5 * device_cus();
+  return P.grid_chunks <= (P.tokens_dev ? kOneLaunchChunks : 20) && groups <= device_cus();
 }
 
 // Partials of one wave per query head: where the chip holds most of the waves at once they
@@ -680,7 +681,7 @@ static bool one_launch_grid(const AttnParams& P) {
 // 1.5 us more than fused multiply-adds (with the fold, 64 / 8 heads: 33 chunks 10.4 -> 8.9
 // us, 192 chunks 18.3 -> 17.3, 256 chunks 19.5 -> 20.4; 512 / 64 heads: 24 chunks 17.1 ->
 // 15.6, 32 chunks 17.1 -> 17.8; 100 tokens of 64 chunks, 64 / 8 heads, 10.5 -> 8.6).
-static bool head_wave_grid(const AttnParams& P) { return (int64_t)P.grid_chunks * P.heads <= 12288; }
+static bool head_wave_grid(const AttnParams& P) { return (int64_t)P.grid_chunks * P.heads <= 48 * device_cus(); }
 
 template <typename T, int G>
 static int launch_attn(const AttnParams& P, int sink_dtype, bool contiguous64, int* counters, hipStream_t st) {

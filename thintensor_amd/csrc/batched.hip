@@ -532,17 +532,6 @@ __global__ __launch_bounds__(64 * WV) void mfma_lds_kernel(MfmaParams P) {
     }
 }
 
-inline int device_cus() {
-  static int cus[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-  if (cus[dev] == 0) {
-    int c = 0;
-    cus[dev] = hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && c > 0 ? c : 256;
-  }
-  return cus[dev];
-}
-
 // Tiles per workgroup (nt <= kMaxNT) and rows per tile (rt <= 16): the fewest rows per
 // workgroup that cover N with one workgroup per CU, cut into as few tiles as hold them.
 struct MfmaPlan {

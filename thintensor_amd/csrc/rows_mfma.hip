@@ -36,7 +36,6 @@
 // MFMAs nor a fragment pipeline across steps moved that, all-zero operands gain 8% (power).
 #include "gemv_impl.h"
 
-#include <atomic>
 #include <type_traits>
 
 using namespace tt;
@@ -419,18 +418,6 @@ __global__ __launch_bounds__(256) void argmax_rows_mfma_kernel(const uint64_t* k
   }
 }
 
-int cu_count() {
-  static std::atomic<int> known[64];
-  int dev = 0, c = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  c = known[dev].load(std::memory_order_relaxed);
-  if (c == 0) {
-    if (hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || c <= 0) c = 256;
-    known[dev].store(c, std::memory_order_relaxed);
-  }
-  return c;
-}
-
 template <Fmt F, int RT, int MT, bool NARROW, bool AM>
 void launch_lpr_rows(int lpr, bool wide, const RowsParams& P, int grid, hipStream_t st) {
   const dim3 g(grid), t(wide ? 512 : 256);
@@ -457,7 +444,7 @@ void launch_lpr_rows(int lpr, bool wide, const RowsParams& P, int grid, hipStrea
 //   * The grid is what the chip holds at once: tiles past it are taken in turn.
 template <Fmt F, bool AM>
 int launch_pass(int lpr, RowsParams P, int64_t keys_per_row, hipStream_t st, int* entries) {
-  const int cus = cu_count();
+  const int cus = device_cus();
   const int rt = P.m <= 16 && P.rows >= 128 * (int64_t)cus ? 2 : 1;
   P.tiles = (P.rows + 16 * rt - 1) / (16 * rt);
   const bool wide = rt == 1 && P.tiles <= cus && lpr >= 32;

@@ -5,6 +5,7 @@
 #include <stdint.h>
 #include <stdarg.h>
 #include <stdio.h>
+#include <atomic>
 #include <string>
 
 #include "../../include/thintensor_hip.h"
@@ -36,6 +37,19 @@ inline int check_launch(const char* what) {
     return TT_ERR_HIP;
   }
   return TT_OK;
+}
+
+// Compute units of the current device.
+inline int device_cus() {
+  static std::atomic<int> known[64];
+  int dev = 0, c = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  c = known[dev].load(std::memory_order_relaxed);
+  if (c == 0) {
+    if (hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || c <= 0) c = 256;
+    known[dev].store(c, std::memory_order_relaxed);
+  }
+  return c;
 }
 
 inline bool aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }
