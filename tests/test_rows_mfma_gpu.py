@@ -137,3 +137,27 @@ def test_fp8_rows_match_single_rows(backend, device, m, rows, cols):
     for t in range(m):
         backend.scaled_matvec(w, scales, x[t], one[t])
     assert torch.equal(out.view(torch.int16), one.view(torch.int16))
+
+
+@pytest.mark.parametrize("m", [3, 4, 7])
+def test_activation_rows_64_mib_apart(backend, device, m):
+    """Row strides past the matrix-core kernel's 32-bit offsets take the GEMV engine, four, two
+    and one rows a launch, with the bits of the same rows side by side."""
+    rows, cols = 3000, 512
+    g = torch.Generator(device=device).manual_seed(m)
+    w, bias = (torch.randn(s, generator=g, device=device).mul_(0.05).half() for s in ((rows, cols), (rows,)))
+    w8 = torch.randn((rows, cols), generator=g, device=device).mul_(100).clamp_(-448, 448).to(torch.float8_e4m3fn)
+    scales = torch.rand(rows, generator=g, device=device) * 0.01 + 1e-3
+    x = torch.randn((m, cols), generator=g, device=device).half()
+    w[rows // 2] = w[rows - 1] = x[m - 1] * 0.25          # a tied maximum of the last row
+    far = torch.empty((m, 1 << 25), device=device, dtype=torch.float16)[:, :cols]
+    far.copy_(x)
+    results = []
+    for a in (far, x):
+        y, y8, logits = (torch.empty((m, rows), device=device, dtype=torch.float16) for _ in range(3))
+        backend.matvec_bias_rows(w, bias, a, y)
+        backend.scaled_batched_matvec(w8, scales, a, y8)
+        tokens = backend.matvec_argmax_batched(w, a, logits)
+        results.append((y.view(torch.int16), y8.view(torch.int16), logits.view(torch.int16), tokens))
+    for got, want in zip(*results):
+        assert torch.equal(got, want)

@@ -604,8 +604,8 @@ int launch_mfma(MfmaParams P, hipStream_t st, const char* what) {
   return rc ? rc : check_launch(what);
 }
 
-// Up to four activation rows per GEMV launch; VALU, bit-exact per row.
-template <Fmt F, SMode SM, typename ST, int ROWS, int L, bool AM>
+// Up to MAXR (two or four) activation rows per GEMV launch; VALU, bit-exact per row.
+template <Fmt F, SMode SM, typename ST, int ROWS, int L, bool AM, int MAXR>
 int launch_rows(GemvParams P, int64_t m_total, int64_t x_row, int64_t out_row, int lpr, hipStream_t st,
                 const char* what, int64_t partial_stride) {
   P.x_slot = x_row;
@@ -615,14 +615,17 @@ int launch_rows(GemvParams P, int64_t m_total, int64_t x_row, int64_t out_row, i
   uint64_t* part0 = P.am_partials;
   for (int64_t m0 = 0; m0 < m_total;) {
     const int64_t left = m_total - m0;
-    const int mr = left >= 4 ? 4 : (left >= 2 ? 2 : 1);
+    const int mr = left >= MAXR ? MAXR : (left >= 2 ? 2 : 1);
     GemvParams Q = P;
     Q.x = x0 + m0 * x_row;
     if (out0) Q.seg[0].out = out0 + m0 * out_row * 2;
     if (AM) Q.am_partials = part0 + m0 * partial_stride;
     int rc;
     switch (mr) {
-      case 4: rc = launch_lpr<F, SM, f16_t, f16_t, ST, ROWS, L, Pro::kLoad, false, 1, 4>(lpr, Q, 1, st, what); break;
+      case 4:
+        if constexpr (MAXR == 4) rc = launch_lpr<F, SM, f16_t, f16_t, ST, ROWS, L, Pro::kLoad, false, 1, 4>(lpr, Q, 1, st, what);
+        else rc = TT_ERR_INVALID;
+        break;
       case 2: rc = launch_lpr<F, SM, f16_t, f16_t, ST, ROWS, L, Pro::kLoad, false, 1, 2>(lpr, Q, 1, st, what); break;
       default: rc = launch_lpr<F, SM, f16_t, f16_t, ST, ROWS, L, Pro::kLoad, false, 1, 1>(lpr, Q, 1, st, what); break;
     }
@@ -690,8 +693,7 @@ int dense_bias_rows_f16(const void* weight, int64_t w_row, const void* bias, con
   P.x = x;
   P.cols = (int)cols;
   const int lpr = tt_gemv_lanes_per_row(cols / 32, 1);
-  return launch_rows<Fmt::kF16W, SMode::kNone, float, 2, 1, false>(P, m, x_row, out_row, lpr, st,
-                                                                         "matvec_bias_rows", 0);
+  return launch_rows<Fmt::kF16W, SMode::kNone, float, 2, 1, false, 4>(P, m, x_row, out_row, lpr, st, "matvec_bias_rows", 0);
 }
 }  // namespace tt
 
@@ -739,7 +741,7 @@ extern "C" int tt_int4_batched_matvec(const void* packed, int64_t w_row_bytes, c
   P.x = x;
   P.cols = (int)cols;
   const int lpr = tt_gemv_lanes_per_row(cols / 32, 4);
-  return launch_rows<Fmt::kInt4Sym, SMode::kGroup, f16_t, 2, 4, false>(P, m, x_row, out_row, lpr, st, what, 0);
+  return launch_rows<Fmt::kInt4Sym, SMode::kGroup, f16_t, 2, 4, false, 2>(P, m, x_row, out_row, lpr, st, what, 0);
 }
 
 extern "C" int tt_scaled_batched_matvec(const void* weight, int64_t w_row_bytes, const float* scales, const void* x,
@@ -773,7 +775,7 @@ extern "C" int tt_scaled_batched_matvec(const void* weight, int64_t w_row_bytes,
   P.x = x;
   P.cols = (int)cols;
   const int lpr = tt_gemv_lanes_per_row(cols / 32, 1);
-  return launch_rows<Fmt::kFp8, SMode::kRow, float, 2, 1, false>(P, m, x_row, out_row, lpr, st, what, 0);
+  return launch_rows<Fmt::kFp8, SMode::kRow, float, 2, 1, false, 4>(P, m, x_row, out_row, lpr, st, what, 0);
 }
 
 extern "C" int64_t tt_matvec_argmax_batched_partials(int64_t m, int64_t rows, int64_t cols) {
@@ -805,8 +807,7 @@ extern "C" int tt_matvec_argmax_batched(const void* weight, int64_t w_row, const
   P.am_partials = partials;
   const int lpr = tt_gemv_lanes_per_row(cols / 32, 1);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  int rc = launch_rows<Fmt::kF16W, SMode::kNone, float, 2, 1, true>(P, m, x_row, logits ? logits_row : 0, lpr, st,
-                                                                    what, per);
+  int rc = launch_rows<Fmt::kF16W, SMode::kNone, float, 2, 1, true, 4>(P, m, x_row, logits ? logits_row : 0, lpr, st, what, per);
   if (rc) return rc;
   hipLaunchKernelGGL(argmax_rows_kernel, dim3((unsigned)m), dim3(256), 0, st, partials, per, m, out_idx, out_val);
   return check_launch(what);
