@@ -521,9 +521,10 @@ int tt_moe_router_topk(const void* logits, int logits_dtype, int64_t experts, in
  * The reference has no batched variant (its kernels take one activation vector and
  * its tensor-core variants broadcast it, triton_kernels.py:596-638); these extend
  * TritonDecodeBackend.int4_scaled_matvec (:4597-4743) and scaled_matvec (:4452-4595)
- * to M rows.  Small M (int4: M < 4, fp8: M < 16) runs the GEMV engine on up to four
- * rows per launch (row m equals the single-row operator bit for bit); from there (up
- * to 64) an MFMA kernel runs whose fp32 sums follow the hardware's order (tolerance
+ * to M rows.  Small M (int4: M < 4, fp8: M < 16): row m equals the single-row operator
+ * bit for bit (the GEMV engine on two rows per launch; fp8 from three rows up to 32 per
+ * pass on the binary32 matrix cores, few weight rows as slots of the single-row kernel);
+ * from there (up to 64) an MFMA kernel runs whose fp32 sums follow the hardware's order (tolerance
  * parity).  cols must be a multiple of 256 up to 8192.  The MFMA path is one launch
  * with no workspace: one workgroup per CU owns a block of weight rows for every
  * activation row, its four waves split K, and their fp32 tiles are summed in a fixed

@@ -157,10 +157,10 @@ def test_rope_table_and_device_position(backend, device):
         assert_f64(from_torch_bits(got), np.concatenate([first, second], axis=1), "rope")
 
 
-@pytest.mark.parametrize("cap", [1100, 1152])  # 1152: whole chunks, contiguous rows -> vector-load kernel
+@pytest.mark.parametrize("cap", [1100, 1152])  # 1152: whole chunks, contiguous rows
 @pytest.mark.parametrize("heads,kv_heads,tokens,sinks", [(32, 8, 513, False), (64, 8, 1025, True), (8, 8, 5, False),
                                                          (32, 8, 64, True), (128, 8, 1100, False),
-                                                         # 64 KV heads x 18 chunks: two chunks per workgroup
+                                                         # 64 KV heads x 18 chunks: partials, then the fold
                                                          (256, 64, 1025, True), (512, 64, 705, False)])
 def test_gqa_attention(backend, device, heads, kv_heads, tokens, sinks, cap):
     D = 64
@@ -400,7 +400,7 @@ def test_unrounded_argmax_matches_binary32_logits(backend, device, rows, cols):
     (16, 16, 1, 64),       # one token, one query head per KV head
     (32, 4, 130, 1024),    # eight query heads per KV head, most of the capacity unused
     (8, 2, 200, 256),      # four heads of 64 (cols 512: 16 lanes per row)
-    (32, 8, 8300, 8320),   # 130 chunks x 8 KV heads > 1024 workgroups: two chunks per workgroup, odd count on the 2nd call
+    (32, 8, 8300, 8320),   # 130 chunks: the count read before the rows, odd on the 2nd call
 ])
 def test_attention_then_int4_matvec(backend, device, heads, kv_heads, tokens, cap):
     """o_proj that combines the attention chunk partials itself: the combined activation

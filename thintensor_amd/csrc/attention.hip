@@ -377,9 +377,10 @@ __global__ __launch_bounds__(64 * G) void attn_kvchunk_kernel(AttnParams P, int*
 // per query head and one workgroup per KV head folding 512 chunks); 512 / 64 x 64, 4096: 46 ->
 // 27; 40 / 10 x 128, 4001: 30.8 -> 14.7; 64 / 8 x 128, 32768: 148 -> 49.5 (2.7 TB/s; both
 // scalar loads before; they are faster only for 20 tokens or fewer, 8 / 8 x 128, 16 tokens:
-// 8.1 against 8.7).  Past a few thousand tokens the partials bound it:
-// about 16 us at 4112 waves, vector and LDS work of about 480 and 130 instructions a wave
-// and the latency of 2 x 64 dependent MFMAs rather than memory.
+// 8.0 against 8.8).  Past a few thousand tokens the partials bound it:
+// 64 / 8 x 64, 16385 tokens: 17 us of partials and 6 of the fold under the profiler; 4112 waves
+// of about 595 vector, 128 matrix and 118 LDS instructions, the matrix cores busy 15% of the
+// time, and the latency of 2 x 64 dependent MFMAs rather than memory.
 typedef float acc4_t __attribute__((ext_vector_type(4)));
 
 template <typename T, int G, int D>
@@ -669,7 +670,7 @@ static int launch_mfma_partials(const AttnParams& P, hipStream_t st) {
 // against 8.7); a count that only the device knows is taken to be half the capacity or more
 // (33 chunks: 64 tokens 6.2 against 7.3 us, 1000 tokens 8.0 against 7.8, all 11.9 against
 // 8.9).  Several workgroups per CU while their fold is short (512 / 64 heads: 9 chunks, 288
-// tokens, 8.5 against 9.8 us, full 11.4 against 11.0; 16 chunks 17.9 against 12.5).
+// tokens, 8.4 against 9.8 us, full 11.3 against 11.0; 16 chunks 17.9 against 12.5).
 static bool one_launch_grid(const AttnParams& P) {
   const int64_t groups = (int64_t)P.grid_chunks * P.kv_heads;
   if (P.grid_chunks <= 10) return 2 * groups <= 5 * device_cus();

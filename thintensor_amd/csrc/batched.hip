@@ -1,10 +1,11 @@
 // Batched small-M dequant GEMM: y[m] = W x[m] for M activation rows.
 //
 //   * M below the fp16 MFMA threshold (int4: 4, fp8: 16): every row has the bits of the
-//     single-row GEMV.  fp8 M >= 3 runs on the binary32 matrix cores (rows_mfma.hip); M = 2,
-//     int4 M = 3 and operands past its 32-bit offsets run the GEMV engine with up to four
-//     activation rows per wave (every weight word decoded once, one fma chain per
-//     activation row); one int4 or fp8 row goes to the single-row kernel itself;
+//     single-row GEMV.  fp8 M >= 3 runs on the binary32 matrix cores (rows_mfma.hip) or, few
+//     weight rows, as slots of the single-row kernel; M = 2, int4 M = 3 and operands past 32-bit
+//     offsets run the GEMV engine with two (four) activation rows per wave (every weight word
+//     decoded once, one fma chain per activation row); one int4 or fp8 row goes to the
+//     single-row kernel itself;
 //   * from the threshold (int4 M >= 4, where the engine's per-row fma chains make it
 //     VALU-bound; fp8 M >= 16): MFMA (mfma_ksplit_kernel below): one workgroup per CU
 //     owns a block of weight rows for all M (<= 64) activation rows, its four waves
@@ -13,9 +14,10 @@
 //     end.  MFMA sums products in a hardware-defined order, so this path matches the
 //     dequantise-then-matmul reference to the stated tolerance, not bit for bit.
 //   * the M-row lm_head argmax and the M-row dense GEMV + bias of a batched decode step
-//     (tt_matvec_bias_rows, fp16) run on the binary32 matrix cores from three rows on, each
-//     row with the bits of the single-row operator; below that the GEMV engine, with one
-//     argmax key per (wave, row) and a finishing kernel that picks each row's token.
+//     (tt_matvec_bias_rows, fp16, unless its weight has few rows) run on the binary32 matrix
+//     cores from three rows on, each row with the bits of the single-row operator; below that
+//     the GEMV engine, with one argmax key per (wave, row) and a finishing kernel that picks
+//     each row's token.
 #include "gemv_impl.h"
 
 #include <type_traits>

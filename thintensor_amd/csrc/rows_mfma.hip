@@ -26,14 +26,16 @@
 // 345 -> 350 us for the 152064 x 5120 head at 16 rows, 43 -> 49 us for an fp8 17920 x 5120
 // matrix.)
 //
-// What bounds it: up to 16 activation rows the weight stream, past it the binary32 matrix
-// rate (130 - 140 TFLOP/s in a loop of these instructions alone).  152064 x 5120 fp16 head
-// with argmax, against one GEMV-engine pass per eight (four, two, one) rows: 4 rows 284 ->
-// 270 us (5.8 TB/s), 8 rows 340 -> 306, 16 rows 677 -> 339, 32 rows 1350 -> 594, 64 rows
-// 2692 -> 1184 us (84 TFLOP/s); fp8 17920 x 5120, 8 rows 47.0 -> 33.9 us, 15 rows 105 ->
-// 38.7 us; fp16 2880 x 4096 + bias, 8 rows 13.8 -> 10.3 us.  Past 16 rows counters show the
-// matrix cores busy 60% of the time; neither the grid, the interleaving of conversions and
-// MFMAs nor a fragment pipeline across steps moved that, all-zero operands gain 8% (power).
+// What bounds it: up to four activation rows the weight stream; up to 16 conversions and
+// matrix issue on top of it (matrix cores busy 29% of the time at 8 rows, 59% at 16, waves
+// waiting to issue 57% and 67% of theirs); past it the binary32 matrix rate (130 - 140 TFLOP/s
+// in a loop of these instructions alone, busy 60% at 32 rows).  152064 x 5120 fp16 head with
+// argmax, against one GEMV-engine pass per eight (four, two, one) rows: 4 rows 276 -> 259 us
+// (6.0 TB/s), 8 rows 339 -> 307, 16 rows 687 -> 341 (4.6 TB/s), 32 rows 1373 -> 603, 64 rows
+// 2765 -> 1213 us (82 TFLOP/s); fp8 17920 x 5120, 8 rows 50.9 -> 34.7 us, 15 rows 110 -> 39
+// us; fp16 2880 x 4096 + bias, 8 rows 15.7 -> 11.3 us.  Neither the grid, the interleaving of
+// conversions and MFMAs nor a fragment pipeline across steps moved the 60%, all-zero operands
+// gain 8% (power).
 #include "gemv_impl.h"
 
 #include <type_traits>
@@ -434,13 +436,15 @@ void launch_lpr_rows(int lpr, bool wide, const RowsParams& P, int grid, hipStrea
 }
 
 // One pass of at most kRowsPass activation rows.
-//   * Up to eight rows run on the 4 x 4 form (16 x 16 would multiply padding: 345 against
-//     335 us for the 152064 x 5120 head at 8 rows, 43 against 38 us for fp8 17920 x 5120).
+//   * Up to eight rows run on the 4 x 4 form (16 x 16 would multiply padding: 337 against
+//     307 us for the 152064 x 5120 head at 8 rows, 335 against 259 at 4, 39 against 35 us for
+//     fp8 17920 x 5120 at 8; the 128256 x 2048 head at 8 rows is the exception, 126 against
+//     134).
 //   * Two weight tiles per wave, their activation operand built once for both, from 128
-//     rows per CU on (8 rows: 332 against 344 us at 152064 weight rows, but 50 against
-//     46 us at 20000, where the last wave of tiles counts more).
-//   * Eight waves per workgroup while there is at most one tile per CU (8 rows: 11.7 -> 10.8
-//     us for 2880 x 4096 fp16, 10.4 -> 9.8 us for 4096 x 5120 fp8; with 320 tiles no gain).
+//     rows per CU on (152064 x 5120: 16 rows 372 us with one, 341 with two, 8 rows 314 and 307;
+//     20000 x 5120, 8 rows, 45 with one and 50 with two: the last turn of tiles counts more).
+//   * Eight waves per workgroup while there is at most one tile per CU (8 rows: 12.3 -> 11.3
+//     us for 2880 x 4096 fp16, 11.1 -> 10.6 us for 4096 x 5120 fp8; with 320 tiles no gain).
 //   * The grid is what the chip holds at once: tiles past it are taken in turn.
 template <Fmt F, bool AM>
 int launch_pass(int lpr, RowsParams P, int64_t keys_per_row, hipStream_t st, int* entries) {

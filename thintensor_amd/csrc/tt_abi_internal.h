@@ -71,16 +71,16 @@ int scaled_slots_fp8(const void* weight, int64_t w_row_bytes, const float* scale
 // rows.  Shapes (cols a multiple of 32) and 16-byte alignment checked by the caller.
 constexpr int kRowsPass = 32;
 // Smallest M of the fp16 GEMVs and of the fp8 GEMM that runs there (same bits as the GEMV
-// engine).  Three rows take the engine two launches (fp16 152064 x 5120 522 us against 263,
-// fp8 17920 x 5120 39 against 24); at two, one launch each, the engine is as fast or faster
-// (268 against 263 us, 18.8 against 21.2).
+// engine).  Three rows take the engine two launches (fp16 152064 x 5120 522 us against 258,
+// fp8 17920 x 5120 39 against 24); at two, one launch each, the head takes 268 us on the engine
+// and 263 here, the fp8 matrix 18.8 and 21.2.
 constexpr int kRowsMfmaMin = 3;
 // Whether the activation rows run sooner as slots of the single-row lean kernel (a grid row
 // each, the same bits): their time grows with rows x m, that of a matrix-core pass of up to 4,
 // 8, 16 or 32 rows hardly does while there are fewer row tiles than CUs.  Break-even of fp16
 // matrices of 2048 to 32768 columns; us as slots against matrix cores: 64 x 5120, 64 rows 5.2
 // against 36.9; 1024 x 5120, 3 rows 6.3 against 8.5, 8 rows 9.2 against 11.4, 16 rows 14.1
-// against 13.3; 1536 x 5120, 4 rows 9.6 against 8.9; 768 x 8192, 32 rows 27 against 29; 2880 x
+// against 13.3; 1536 x 5120, 4 rows 9.6 against 8.9; 768 x 8192, 32 rows 27 against 28; 2880 x
 // 5120, 8 rows 31 against 12; a fifth earlier where the slots' weight reads miss the L2s
 // (1280 x 32768, 4 rows 46 against 34).  (fp8 breaks even later: 2048 x 5120, 8 rows 1.2 times
 // as fast as slots, 2880 x 5120 0.85 times.)
